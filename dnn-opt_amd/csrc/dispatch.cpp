@@ -33,9 +33,11 @@
 //     the CUs, with a separate reduce kernel once the split count is large.
 //   * int8 (B as N x K): the row-dot kernel (v_dot4) for M <= 4; 16 x 16
 //     MFMA tiles with k split over the waves of a workgroup for M <= 16;
-//     32 x 32 tiles staged through LDS (256-byte k-blocks) above that (4-byte
-//     aligned rows), split-k only when the tiles leave more than half of the
-//     CUs idle.
+//     tiles copied into LDS by the memory unit above that (4-byte aligned
+//     rows), 32 x 32 to 64 x 64 by a rule or, where a cost model (kS8Model)
+//     is 5% ahead of it, another tile or split, up to k_pp.hip's 256 x 256.
+//   * bf16 storage with more than 64 rows and K a multiple of 8: k_pp.hip's
+//     tiles where their cost model is ahead of the other tiles'.
 //   The LDS-staged tile and k-split of bf16 storage above M = 128, and of
 //   fp32 inputs above M = 64, come from a fitted cost model (pick_tile) when
 //   it beats the rule by 5%; the fp32 register tile and k-split (A stored
@@ -426,6 +428,74 @@ static TilePick pick_lds_tile(const LdsModel& md, int tb, int M, int N, int K, i
     return best;
 }
 
+// Whole-workgroup cost model of the LDS-DMA tiles that run one or two to a
+// CU: k_pp.hip's tiles (bf16 storage and int8), and the other int8 LDS-DMA
+// tiles.  A launch gives each CU per = ceil(tiles splits / CUs) workgroups;
+// with one workgroup to a CU each takes fill + blocks t1 (fill: first copies,
+// epilogue, its share of C), with two resident a pair takes fill + blocks t2;
+// a launch takes a fixed time and no less than its bytes at the fitted rate;
+// a k-split adds a fixed time plus its partials, written and read.
+//   bf16: 160 shapes (M = 65..4096, N = 512..11008, K = 512..4608, both B
+//   layouts; 7 tiles, 1 to 4 splits, 2431 points): median error 3.4%, 90%
+//   within 10%.
+//   int8: 180 shapes (M = 17..4096, same N and K; 10 tiles, 1 to 4 splits):
+//   median error 6%, 90% within 16%.
+struct WgFit {
+    int cfg, occ;
+    double fill, t1, t2;
+};
+struct WgModel {
+    const WgFit* fits;
+    int n;
+    int es;  // operand bytes per element
+    double launch_us, split_us, partial_ps, hbm_ps;
+};
+static const WgFit kBf16PPFit[] = {
+    {51, 1, 8.285, 1.107, 0.0},   {52, 1, 6.806, 1.043, 0.0},   {53, 1, 4.990, 0.740, 0.0},   {54, 2, 3.143, 0.519, 0.864},
+    {55, 1, 5.115, 0.801, 0.0},   {56, 2, 4.429, 0.701, 1.491}, {57, 2, 3.169, 0.649, 0.968},
+};
+static const WgFit kS8Fit[] = {
+    {22, 2, 1.520, 0.196, 0.375}, {23, 2, 1.700, 0.366, 0.649}, {29, 2, 2.147, 0.230, 0.460}, {30, 1, 9.191, 1.099, 0.0},
+    {31, 1, 7.616, 1.065, 0.0},   {32, 1, 5.852, 0.762, 0.0},   {33, 2, 4.134, 0.526, 1.133}, {34, 1, 6.027, 0.821, 0.0},
+    {35, 2, 5.293, 0.712, 1.539}, {36, 2, 4.191, 0.661, 1.222},
+};
+static const WgModel kBf16PPModel{kBf16PPFit, (int)(sizeof kBf16PPFit / sizeof kBf16PPFit[0]), 2, 3.007, 2.543, 0.152, 0.439};
+static const WgModel kS8Model{kS8Fit, (int)(sizeof kS8Fit / sizeof kS8Fit[0]), 1, 1.5, 2.801, 0.198, 0.381};
+
+static double wg_cost(const WgModel& md, const WgFit& f, int bm, int bn, int kb, long long s, int M, int N, int K,
+                      long long cus) {
+    const long long tiles = ceil_div(M, bm) * ceil_div(N, bn), blocks = ceil_div(ceil_div(K, kb), s);
+    const long long per = ceil_div(tiles * s, cus);
+    const double one = f.fill + (double)blocks * f.t1;
+    const double core = f.occ == 1 ? (double)per * one
+                                   : (double)(per / 2) * (f.fill + (double)blocks * f.t2) + (double)(per % 2) * one;
+    const double bytes = (double)md.es * ((double)M * K + (double)K * N) + 4.0 * M * N;
+    double us = md.launch_us + std::max(core, bytes * md.hbm_ps * 1e-6);
+    if (s > 1) us += md.split_us + 2.0 * (double)s * tiles * bm * bn * 4 * md.partial_ps * 1e-6;
+    return us;
+}
+
+// The model's best configuration and split (1, 2 or 4, while the workgroups
+// stay within about one round: more splits than that only add partials).
+// shape(cfg, &bm, &bn, &kb) says whether a configuration may be used.
+template <class Shape>
+static TilePick best_wg_tile(const WgModel& md, int M, int N, int K, Shape shape) {
+    const long long cus = num_cus();
+    TilePick best{0, 0, 0.0};
+    for (int i = 0; i < md.n; ++i) {
+        const WgFit& f = md.fits[i];
+        int bm = 0, bn = 0, kb = 0;
+        if (!shape(f.cfg, &bm, &bn, &kb)) continue;
+        const long long tiles = ceil_div(M, bm) * ceil_div(N, bn), nblk = ceil_div(K, kb);
+        for (long long s : {1, 2, 4}) {
+            if (s > 1 && (s > nblk || s > max_splits() || tiles * s > cus + cus / 8)) break;
+            const double us = wg_cost(md, f, bm, bn, kb, s, M, N, K, cus);
+            if (best.s == 0 || us < best.us) best = TilePick{f.cfg, s, us};
+        }
+    }
+    return best;
+}
+
 // k-splits of an fp32 register-tile launch by the occupancy rule: split k
 // when the tiles give fewer workgroups than waves_per_cu() waves on every CU.
 static long long reg_tile_splits(int cfg, int M, int N, int K) {
@@ -588,11 +658,27 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
                 cfg = pick.cfg;
                 model_splits = pick.s;
             }
+            // bf16 storage, more than 64 rows: k_pp.hip's tiles where their
+            // model puts them ahead of that choice's.  (Their k-contiguous
+            // rows are cut off at whole 16-byte chunks, hence K % 8.)
+            if (mode == kTileBF16 && M > 64 && K % 8 == 0 && tall_ok) {
+                const TilePick pp = best_wg_tile(kBf16PPModel, M, N, K, [&](int k, int* bm_, int* bn_, int* kb_) {
+                    const TileConfig t = tile_config(k);
+                    *bm_ = t.wm * t.mt * 16;
+                    *bn_ = t.wn * t.nt * 16;
+                    *kb_ = t.kblk;
+                    return true;
+                });
+                if (pp.s > 0 && pick.us > 0.0 && pp.us < pick.us) {
+                    cfg = pp.cfg;
+                    model_splits = pp.s;
+                }
+            }
         }
         const bool forced_dma = forced_cfg >= kTileFirstDma && forced_cfg < kTileF32Few;
         if (((forced_cfg >= kTileFirstLds && forced_cfg < kTileF32Few) || forced_cfg == kTileBF16Tb48 ||
              forced_cfg == kTileBF16Tb48Few || forced_cfg == kTileBF16Dma4w ||
-             (forced_cfg == kTileF2BTall && tall_ok)) &&
+             (tile_pp(forced_cfg) && mode == kTileBF16 && K % 8 == 0 && tall_ok) || (forced_cfg == kTileF2BTall && tall_ok)) &&
             ((!forced_dma && forced_cfg != kTileBF16Dma4w) || mode == kTileBF16))
             cfg = forced_cfg;
     } else if (mode == kTileF32 && N <= 16) {
@@ -712,8 +798,8 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
     // for the LDS-DMA tiles (tunable TILE_TICKET = 1): the last workgroup to
     // finish a tile adds the others' partials.
     const bool dma_ticket = tunable(kTuneTileTicket) == 1;
-    const bool dma = (cfg >= kTileFirstDma && cfg < kTileF32Few) || cfg == kTileBF16Dma4w;  // LDS-DMA tiles
-    const bool ticket_ok = !lds || (dma_ticket && dma);
+    const bool dma = (cfg >= kTileFirstDma && cfg < kTileF32Few) || cfg == kTileBF16Dma4w || tile_pp(cfg);  // LDS-DMA tiles
+    const bool ticket_ok = !lds || (dma_ticket && dma && !tile_pp(cfg));
     // Split sums: fp32 tiles (register and LDS-DMA) let the tile's
     // last-arriving workgroup add up to 8 splits' partials (one kernel; its
     // threads read the partial block in 16-byte pieces, 8 in flight each),
@@ -736,6 +822,16 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
     return DNNOPT_OK;
 }
 
+// k-splits of an LDS-staged int8 launch by the occupancy rule: k is split only
+// where the tiles leave more than half of the CUs idle.
+static long long s8_rule_splits(int cfg, int M, int N, int K) {
+    const S8Config c = s8_config(cfg);
+    const long long tiles = ceil_div(M, c.wm * c.mt * 16) * ceil_div(N, c.wn * c.nt * 16), cus = num_cus();
+    const long long nblk = ceil_div(K, c.kblk > 0 ? c.kblk : 128);
+    if (tiles * 2 >= cus) return 1;
+    return std::min<long long>({ceil_div(cus, tiles), std::max<long long>(1, nblk / 2), (long long)max_splits()});
+}
+
 static int plan_s8_kernels(int epi, int M, int N, int K, Launch* L, bool lds_ok, int lda, int ldb, int ldc) {
     *L = Launch{};
     if (ldc <= 0) ldc = N;
@@ -750,23 +846,46 @@ static int plan_s8_kernels(int epi, int M, int N, int K, Launch* L, bool lds_ok,
         plan_rowdot(2 + (epi ? 1 : 0), M, N, K, lda > 0 ? lda : K, ldb > 0 ? ldb : K, L) == DNNOPT_OK)
         return DNNOPT_OK;
     *L = Launch{};
-    const int forced_splits = tunable(kTuneS8Splits);
     // M <= 16: 16 x 16 tiles with k split over the 8 waves of a workgroup
     // (one launch, no partial sums).  Larger M: operands copied into LDS by
-    // the memory unit (LDS DMA), the largest of 64 x 64 (4 stages of
-    // 128-byte blocks), 64 x 32 (3 stages of 256 bytes) and 32 x 32 (4
-    // stages of 256 bytes) that still gives every CU a tile.  Measured (us,
-    // against the register-staged 32 x 32 LDS kernel): 128 x 4096 x 4096
-    // 11.2 vs 12.6, 128 x 2048 x 4096 7.9 vs 9.6, 64 x 4096 x 4096 8.8 vs
-    // 10.2, 256 x 4096 x 4096 13.9 vs 21.7, 128 x 8192 x 4096 16.1 vs 22.5.
+    // the memory unit (LDS DMA).  The rule is the largest of 64 x 64 (4 stages
+    // of 128-byte blocks), 64 x 32 (3 stages of 256 bytes) and 32 x 32 (4
+    // stages of 256 bytes) that still gives every CU a tile, k split where
+    // even 32 x 32 tiles leave half of the CUs idle.  Where the cost model
+    // (kS8Model) puts one of these, or above 64 rows one of k_pp.hip's tiles,
+    // with another split 5% ahead of it, that one (measured, us: 100 x 940 x
+    // 2752 8.6 -> 5.9 (no split), 1296 x 4776 x 1280 23.4 -> 15.9 and 1024 x
+    // 11008 x 4096 100.1 -> 48.9 (k_pp.hip)).
     int cfg = 5;
+    long long model_splits = 0;
+    const int forced_splits = tunable(kTuneS8Splits);
+    const bool pp_ok = K % 16 == 0 && 256LL * ldc * 4 < 0x7FFFFFFFll;
     if (M > 16) {
         const long long cus_ = num_cus();
         if (ceil_div(M, 64) * ceil_div(N, 64) >= cus_) cfg = 29;
         else if (ceil_div(M, 64) * ceil_div(N, 32) >= cus_) cfg = 23;
         else cfg = 22;
+        const auto shape = [&](int k, int* bm_, int* bn_, int* kb_) {
+            if (k >= kS8PPFirst && (!pp_ok || M <= 64)) return false;
+            const S8Config t = s8_config(k);
+            *bm_ = t.wm * t.mt * 16;
+            *bn_ = t.wn * t.nt * 16;
+            *kb_ = t.kblk;
+            return true;
+        };
+        int bm0 = 0, bn0 = 0, kb0 = 0;
+        shape(cfg, &bm0, &bn0, &kb0);
+        const WgFit* def = nullptr;
+        for (const WgFit& f : kS8Fit)
+            if (f.cfg == cfg) def = &f;
+        const double def_us = wg_cost(kS8Model, *def, bm0, bn0, kb0, s8_rule_splits(cfg, M, N, K), M, N, K, cus_);
+        const TilePick pick = best_wg_tile(kS8Model, M, N, K, shape);
+        if (forced_cfg < 0 && pick.us < 0.95 * def_us) {
+            cfg = pick.cfg;
+            model_splits = pick.s;
+        }
     }
-    if (forced_cfg >= 0 && forced_cfg < s8_config_count()) cfg = forced_cfg;
+    if (forced_cfg >= 0 && forced_cfg < s8_config_count() && (forced_cfg < kS8PPFirst || pp_ok)) cfg = forced_cfg;
     if (cfg >= kS8FirstLds && !lds_ok) cfg = M <= 16 ? 5 : (M >= 128 ? 3 : 2);
     const bool lds = cfg >= kS8FirstLds;
     const bool dma = cfg >= kS8FirstDma;
@@ -779,8 +898,7 @@ static int plan_s8_kernels(int epi, int M, int N, int K, Launch* L, bool lds_ok,
     const long long cus = num_cus();
     long long s = 1;
     if (lds) {
-        if (tiles * 2 < cus) s = std::min<long long>({ceil_div(cus, tiles), std::max<long long>(1, nblk / 2),
-                                                      (long long)max_splits()});
+        s = model_splits > 0 ? model_splits : s8_rule_splits(cfg, M, N, K);
     } else {
         const long long target_wgs = cus * waves_per_cu() / waves_per_wg;
         if (tiles < target_wgs) {

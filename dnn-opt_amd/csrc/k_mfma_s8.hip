@@ -723,6 +723,14 @@ static const S8Config kS8Configs[] = {
     {2, 1, 2, 2, 1, 4, 256},  // 27: 64 x 32, 4 stages
     {2, 1, 2, 2, 1, 4, 128},  // 28: 64 x 32, 4 stages of 128-byte blocks
     {2, 2, 2, 2, 1, 4, 128},  // 29: 64 x 64, 4 stages of 128-byte blocks
+    // k_pp.hip: {MT, NT, WM, WN, 1, stages, k bytes per block}
+    {8, 4, 2, 4, 1, 2, 128},  // 30: 256 x 256
+    {8, 3, 2, 4, 1, 2, 128},  // 31: 256 x 192
+    {8, 2, 2, 4, 1, 2, 128},  // 32: 256 x 128
+    {4, 2, 2, 4, 1, 2, 128},  // 33: 128 x 128
+    {4, 4, 2, 4, 1, 2, 128},  // 34: 128 x 256
+    {4, 3, 2, 4, 1, 2, 128},  // 35: 128 x 192
+    {8, 1, 2, 4, 1, 2, 128},  // 36: 256 x 64
 };
 
 int s8_config_count() { return (int)(sizeof(kS8Configs) / sizeof(kS8Configs[0])); }
@@ -776,6 +784,27 @@ hipError_t launch_s8_q8b(dim3 grid, const S8Args& a, hipStream_t s) {
 hipError_t launch_mfma_s8(int cfg_idx, int epi, int aligned, dim3 grid, const S8Args& a, hipStream_t s) {
     if (cfg_idx < 0 || cfg_idx >= s8_config_count()) return hipErrorInvalidValue;
     if (cfg_idx >= kS8FirstLds && !aligned) return hipErrorInvalidValue;
+    if (cfg_idx >= kS8PPFirst) {
+        PPArgs q{};
+        q.A = a.A;
+        q.B = a.B;
+        q.C = a.C;
+        q.part = a.part;
+        q.lda = a.lda;
+        q.ldb = a.ldb;
+        q.ldc = a.ldc;
+        q.M = a.M;
+        q.N = a.N;
+        q.K = a.K;
+        q.alpha = a.alpha;
+        q.beta = a.amax ? a.beta : 0.0f;
+        q.splits = a.splits;
+        q.tiles_n = a.tiles_n;
+        q.tiles_m = a.tiles_m;
+        q.scale = a.scale;
+        q.amax = a.amax;
+        return launch_pp(1, cfg_idx - kS8PPFirst, 1, epi, grid, q, s);
+    }
     if (epi) return aligned ? launch_s8_cfg<1, 1>(cfg_idx, grid, a, s) : launch_s8_cfg<1, 0>(cfg_idx, grid, a, s);
     return aligned ? launch_s8_cfg<0, 1>(cfg_idx, grid, a, s) : launch_s8_cfg<0, 0>(cfg_idx, grid, a, s);
 }

@@ -1341,6 +1341,14 @@ static const TileConfig kTileConfigs[] = {
     {1, 2, 2, 1, 1, 3, 32},   // 48: 32 x 32, 2 waves of 16 x 32
     {2, 2, 2, 2, 1, 3, 32},   // 49: 64 x 64, 4 waves of 32 x 32
     {1, 2, 2, 2, 1, 3, 32},   // 50: 32 x 64, 4 waves of 16 x 32
+    // bf16 storage, k_pp.hip: {MT, NT, WM, WN, 1, stages, k per block}
+    {8, 4, 2, 4, 1, 2, 64},   // 51: 256 x 256
+    {8, 3, 2, 4, 1, 2, 64},   // 52: 256 x 192
+    {8, 2, 2, 4, 1, 2, 64},   // 53: 256 x 128
+    {4, 2, 2, 4, 1, 2, 64},   // 54: 128 x 128
+    {4, 4, 2, 4, 1, 2, 64},   // 55: 128 x 256
+    {4, 3, 2, 4, 1, 2, 64},   // 56: 128 x 192
+    {8, 1, 2, 4, 1, 2, 64},   // 57: 256 x 64
 };
 
 int tile_config_count() { return (int)(sizeof(kTileConfigs) / sizeof(kTileConfigs[0])); }
@@ -1397,6 +1405,26 @@ hipError_t launch_tile(int mode, int cfg_idx, int ta, int tb, int al, dim3 grid,
     if (mode != kTileF32 && (ta || (tb && mode != kTileBF16))) return hipErrorInvalidValue;
     if (cfg_idx == kTileKOuter) return mode == kTileF32 && ta && !tb ? launch_kouter_f32(grid, a, s) : hipErrorInvalidValue;
     if (cfg_idx < 0 || cfg_idx >= tile_config_count()) return hipErrorInvalidValue;
+    if (tile_pp(cfg_idx)) {
+        if (mode != kTileBF16 || !al) return hipErrorInvalidValue;
+        PPArgs q{};
+        q.A = a.A;
+        q.B = a.B;
+        q.C = a.C;
+        q.part = a.part;
+        q.lda = a.lda;
+        q.ldb = a.ldb;
+        q.ldc = a.ldc;
+        q.M = a.M;
+        q.N = a.N;
+        q.K = a.K;
+        q.alpha = a.alpha;
+        q.beta = a.beta;
+        q.splits = a.splits;
+        q.tiles_n = a.tiles_n;
+        q.tiles_m = a.tiles_m;
+        return launch_pp(0, cfg_idx - kTilePPFirst, tb, 0, grid, q, s);
+    }
     const TileConfig c = kTileConfigs[cfg_idx];
     const dim3 blk(c.wm * c.wn * c.kw * 64);
     if (cfg_idx >= kTileFirstLds && !al) return hipErrorInvalidValue;

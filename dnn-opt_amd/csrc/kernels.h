@@ -163,6 +163,9 @@ constexpr int kS8FirstLds = 10;
 // vector memory unit's LDS path (no register staging); same requirements
 // and tile order as the LDS-staged ones, depth = stages.
 constexpr int kS8FirstDma = 21;
+// Configurations from this index on are launch_pp's (k_pp.hip), in its order:
+// K a multiple of 16, 256 ldc 4 < 2^31.
+constexpr int kS8PPFirst = 30;
 // Index into the table of built int8 configurations.
 int s8_config_count();
 S8Config s8_config(int idx);
@@ -254,6 +257,10 @@ constexpr int kTileF2BTall = 40;
 // 32 or 64 rows by 64 columns (B stored K x N or N x K), and from
 // kTileF32DmaTbFirst by 32 columns (B stored N x K only).
 constexpr int kTileF32DmaFirst = 41, kTileF32DmaTbFirst = 48, kTileF32DmaLast = 50;
+// bf16 storage, two wave groups taking turns (k_pp.hip): configuration
+// kTilePPFirst + i is launch_pp's i.  K a multiple of 8, 256 ldc 4 < 2^31.
+constexpr int kTilePPFirst = 51, kTilePPLast = 57;
+constexpr bool tile_pp(int cfg) { return cfg >= kTilePPFirst && cfg <= kTilePPLast; }
 constexpr bool tile_f32_dma(int cfg) { return cfg >= kTileF32DmaFirst && cfg <= kTileF32DmaLast; }
 // k per LDS block of an LDS-staged configuration: its kblk (or
 // DNNOPT_LDS_KB) when both stages fit in 128 KiB of LDS, else 64.
@@ -271,6 +278,24 @@ hipError_t launch_kouter_f32(dim3 grid, const TileArgs& a, hipStream_t s);
 // boundaries (matters for bf16 storage).
 hipError_t launch_tile(int mode, int cfg_idx, int transA, int transB, int aligned, dim3 grid,
                        const TileArgs& a, hipStream_t s);
+
+// ---------------------------------------------------------------- large tiles, two wave groups
+// k_pp.hip: bf16 storage (dt 0; B stored K x N, or N x K with tb) and int8
+// (dt 1, B stored N x K).  grid = (xcd_grid(tiles_n, tiles_m), 1, splits).
+struct PPArgs {
+    const void* A;
+    const void* B;
+    void* C;      // float*, or int32_t* (dt 1, epi 0)
+    void* part;   // [splits][tiles][BM*BN] (splits > 1; a reduce kernel follows)
+    int lda, ldb, ldc;
+    int M, N, K;
+    float alpha, beta;
+    int splits;
+    int tiles_n, tiles_m;
+    const float* scale;    // dt 1, epi 1: as S8Args
+    const unsigned* amax;
+};
+hipError_t launch_pp(int dt, int cfg, int tb, int epi, dim3 grid, const PPArgs& a, hipStream_t s);
 
 // ---------------------------------------------------------------- last resort
 // dnnopt_wide (k_wide.hip): any layout and size with 64-bit addressing, for
