@@ -37,7 +37,7 @@
 //     rows), 32 x 32 to 64 x 64 by a rule or, where a cost model (kS8Model)
 //     is 5% ahead of it, another tile or split, up to k_pp.hip's 256 x 256.
 //   * bf16 storage with more than 64 rows and K a multiple of 8: k_pp.hip's
-//     tiles where their cost model is ahead of the other tiles'.
+//     tiles where their cost model is 5% ahead of the other tiles.
 //   The LDS-staged tile and k-split of bf16 storage above M = 128, and of
 //   fp32 inputs above M = 64, come from a fitted cost model (pick_tile) when
 //   it beats the rule by 5%; the fp32 register tile and k-split (A stored
@@ -659,7 +659,7 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
                 model_splits = pick.s;
             }
             // bf16 storage, more than 64 rows: k_pp.hip's tiles where their
-            // model puts them ahead of that choice's.  (Their k-contiguous
+            // model puts them 5% ahead of that choice's.  (Their k-contiguous
             // rows are cut off at whole 16-byte chunks, hence K % 8.)
             if (mode == kTileBF16 && M > 64 && K % 8 == 0 && tall_ok) {
                 const TilePick pp = best_wg_tile(kBf16PPModel, M, N, K, [&](int k, int* bm_, int* bn_, int* kb_) {
@@ -669,7 +669,7 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
                     *kb_ = t.kblk;
                     return true;
                 });
-                if (pp.s > 0 && pick.us > 0.0 && pp.us < pick.us) {
+                if (pp.s > 0 && pick.us > 0.0 && pp.us < 0.95 * pick.us) {
                     cfg = pp.cfg;
                     model_splits = pp.s;
                 }
