@@ -359,6 +359,21 @@ static int gemm_bf16_common(int fp32_inputs, int M, int N, int K, float alpha, c
         return run_wide(fp32_inputs ? kTileF2B : kTileBF16, 0, 0, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, s);
     if (L.family == DNNOPT_K_SKINNY_BF16 || L.family == DNNOPT_K_SKINNY_F2B)
         return run_skinny(L, A, lda, 1, B, ldb, C, ldc, M, N, K, alpha, beta, s);
+    Bf16Copies cp{};
+    if (fp32_inputs && plan_bf16_copies(L, M, N, K, lda, ldb, ldc, &cp)) {
+        // Operands rounded once into workspace (k padded with zeros to a
+        // multiple of 8) ahead of the tiles.  Without the workspace (under
+        // capture, or when memory is short) the tiles below round both while
+        // staging.
+        if (char* ws = static_cast<char*>(optional_workspace(s, cp.bytes, kSlotBf16))) {
+            uint16_t *ca = reinterpret_cast<uint16_t*>(ws), *cb = reinterpret_cast<uint16_t*>(ws + cp.a_bytes);
+            st = finish_launch(launch_bf16_copy(static_cast<const float*>(A), lda, static_cast<const float*>(B), ldb, M,
+                                                N, K, ca, cp.lda, cp.both ? cb : nullptr, cp.ldb, cp.K, s));
+            if (st != DNNOPT_OK) return st;
+            return run_tile(cp.L, 0, 0, ca, cp.lda, cp.both ? static_cast<const void*>(cb) : B, cp.both ? cp.ldb : ldb, C, ldc,
+                            M, N, cp.K, alpha, beta, s);
+        }
+    }
     return run_tile(L, 0, 0, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, s);
 }
 

@@ -600,6 +600,7 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
                      (transB ? ((long long)(N + 128) * ldb + K) : ((long long)K * ldb + N)) * es < 0x7FFFFFFFll &&
                      (long long)128 * ldc * 4 < 0x7FFFFFFFll;
     int cfg;
+    double est_us = 0.0;         // its estimate
     long long model_splits = 0;  // the cost model's split count
     const int forced_cfg = tunable(kTuneTileCfg);
     if (lds) {
@@ -654,6 +655,7 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
             const TilePick pick = mode == kTileBF16
                                       ? pick_lds_tile(kBf16Model, transB ? 1 : 0, M, N, K, cfg, def_s, 0.10, false)
                                       : pick_lds_tile(kF2BModel, 0, M, N, K, cfg, def_s, 0.05, tall_ok);
+            est_us = pick.us;
             if (pick.s > 0) {
                 cfg = pick.cfg;
                 model_splits = pick.s;
@@ -672,6 +674,7 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
                 if (pp.s > 0 && pick.us > 0.0 && pp.us < 0.95 * pick.us) {
                     cfg = pp.cfg;
                     model_splits = pp.s;
+                    est_us = pp.us;
                 }
             }
         }
@@ -786,6 +789,7 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
     if (tm > 65535 || s > 65535 || tn * tm > 0x7FFFFFF0ll) return DNNOPT_ERR_UNSUPPORTED;
     L->mode = mode;
     L->cfg = cfg;
+    L->est_us = est_us;
     L->bm = bm;
     L->bn = bn;
     L->tn = (int)tn;
@@ -1122,6 +1126,80 @@ int plan_bf16(int fp32_inputs, int M, int N, int K, int lda, int ldb, Launch* L,
     const int st = plan_bf16_kernels(fp32_inputs, M, N, K, lda, ldb, L, transB, ldc);
     if (st == DNNOPT_ERR_UNSUPPORTED) plan_wide(M, N, L);
     return st == DNNOPT_ERR_UNSUPPORTED ? DNNOPT_OK : st;
+}
+
+// Tiles of a bf16 A and an fp32 B (kTileA16): 128 x 96 with 128 k per block,
+// 256 x 96 with 64, 1 or 2 k-splits (40 shapes, M = 34..2048, N = 768..11008,
+// K = 768..4096, 143 points: median error 5%, 90% within 12%).
+static const WgFit kA16Fit[] = {{20, 1, 3.505, 1.426, 0.0}, {kTileF2BTall, 1, 3.243, 1.049, 0.0}};
+static const WgModel kA16Model{kA16Fit, 2, 0, 3.812, 2.503, 0.152, 0.0};
+
+// Rounding operands once, into workspace, ahead of the tiles (6 bytes of
+// traffic per element at 6.3 TB/s) against tiles that round every element each
+// time they stage it.  A alone costs one short launch and halves the bytes of
+// A every column of tiles reads; both operands cost a pass over B and gain the
+// bf16-storage tiles' rate, which pays from many hundreds of rows.  Measured
+// (MI355X, us, direct / A / both): 256 x 11008 x 4096 73.1 / 64.1 / 80, 512 x
+// 11008 x 4096 107.8 / 87.4 / 108.6, 1024 x 11008 x 4096 196.5 / 161.1 / 146,
+// 1632 x 4352 x 3520 142.5 / 120.5 / 83.4, 300 x 1001 x 1003 10.5 / 17.7 / -.
+// The direct tiles run at 0.9 of their model's times (0.77..1.16 on those
+// shapes; the fit predates their raw register ring); the other two have to be
+// 5% and 10% ahead.
+bool plan_bf16_copies(const Launch& direct, int M, int N, int K, int lda, int ldb, int ldc, Bf16Copies* out) {
+    if (ldc <= 0) ldc = N;
+    if (direct.est_us <= 0.0 || M <= 64 || (long long)lda * 16 >= 0x7FFFFFFFll || (long long)ldb * 16 >= 0x7FFFFFFFll)
+        return false;
+    const long long k8 = ((long long)K + 7) & ~7ll, n8 = ((long long)N + 7) & ~7ll;
+    const size_t a = ((size_t)M * k8 * 2 + 255) & ~(size_t)255, b = (size_t)k8 * n8 * 2;
+    if (k8 > 0x7FFFFFF0ll || n8 > 0x7FFFFFF0ll) return false;
+    out->lda = (int)k8;
+    double best = 0.90 * direct.est_us;
+    bool found = false;
+    // The direct plan's spans (B, and A in fp32) fit 32-bit offsets; so must
+    // 256 rows of C.
+    if (a <= kOptionalBytes && 256LL * ldc * 4 < 0x7FFFFFFFll) {
+        const TilePick t = best_wg_tile(kA16Model, M, N, K, [&](int k, int* bm_, int* bn_, int* kb_) {
+            const TileConfig c = tile_config(k);
+            *bm_ = c.wm * c.mt * 16;
+            *bn_ = c.wn * c.nt * 16;
+            *kb_ = tile_lds_bk(*bm_, *bn_, c.kblk);
+            return true;
+        });
+        const double us = t.us + (double)M * K * 6e-6 / 6.3;
+        if (t.s > 0 && us < 0.95 * best) {
+            const TileConfig c = tile_config(t.cfg);
+            Launch& L = out->L;
+            L = Launch{};
+            L.mode = kTileA16;
+            L.cfg = t.cfg;
+            L.bm = c.wm * c.mt * 16;
+            L.bn = c.wn * c.nt * 16;
+            L.tn = (int)ceil_div(N, L.bn);
+            L.tm = (int)ceil_div(M, L.bm);
+            L.grid = dim3((unsigned)xcd_grid(L.tn, L.tm), 1, (unsigned)t.s);
+            L.defer_reduce = t.s > 1 ? 1 : 0;
+            L.part_bytes = t.s > 1 ? (size_t)t.s * L.tn * L.tm * L.bm * L.bn * sizeof(float) : 0;
+            out->both = false;
+            out->K = K;
+            out->a_bytes = out->bytes = a;
+            best = us;
+            found = true;
+        }
+    }
+    const double copy_us = 5.0 + ((double)M * K + (double)K * N) * 6e-6 / 6.3;
+    Launch two;
+    if (a + b <= kOptionalBytes && copy_us < best &&
+        plan_bf16(0, M, N, (int)k8, (int)k8, (int)n8, &two, 0, ldc) == DNNOPT_OK && two.est_us > 0.0 &&
+        copy_us + two.est_us < 0.9 * best) {
+        out->L = two;
+        out->both = true;
+        out->K = (int)k8;
+        out->ldb = (int)n8;
+        out->a_bytes = a;
+        out->bytes = a + b;
+        found = true;
+    }
+    return found;
 }
 
 }  // namespace dnnopt_hip

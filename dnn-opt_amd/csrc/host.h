@@ -26,6 +26,13 @@ constexpr int kMaxTickets = 4096;  // ticket slots, kTicketStride words each
 constexpr size_t kTicketBytes = (size_t)kMaxTickets * kTicketStride * sizeof(unsigned);
 int get_workspace(hipStream_t s, size_t part_bytes, void** part, unsigned** tickets, int slot = 0);
 
+// Scratch of a slot for an optional faster route, without tickets and kept
+// like get_workspace's, at most kOptionalBytes per (device, stream).  nullptr
+// while the stream is being captured and when memory is short: the caller
+// takes its other route.
+constexpr size_t kOptionalBytes = (size_t)256 << 20;
+void* optional_workspace(hipStream_t s, size_t bytes, int slot);
+
 // Serialises the calls that enqueue work on one stream of one device (the
 // current device).  Every entry point that may take workspace holds it from
 // planning until its last launch is enqueued, so that
@@ -73,6 +80,7 @@ struct Launch {
     size_t part_bytes = 0;
     int tickets = 0;
     int defer_reduce = 0;
+    double est_us = 0.0;  // LDS-staged tiles: the cost models' time (0 = none made)
 };
 
 // Split-k reduction strategy (tunable SPLIT_REDUCE): 0 = last-arriving
@@ -158,9 +166,22 @@ int plan_sgemm(int transA, int transB, int M, int N, int K, int lda, int ldb, La
 // transB: B stored N x K, bf16 storage only).
 int plan_bf16(int fp32_inputs, int M, int N, int K, int lda, int ldb, Launch* L, int transB = 0, int ldc = 0);
 
+// The fp32-input bf16 GEMM with operands rounded to bf16 into workspace ahead
+// of the tiles: A alone (k_pp.hip's tiles round the fp32 B) or both (the
+// bf16-storage tiles).  Row strides and k of the copies in elements; false
+// where the tiles that round while staging are estimated faster, or the
+// copies may not be made.
+struct Bf16Copies {
+    bool both;
+    int lda, ldb, K;
+    size_t a_bytes, bytes;
+    Launch L;
+};
+bool plan_bf16_copies(const Launch& direct, int M, int N, int K, int lda, int ldb, int ldc, Bf16Copies* out);
+
 // Workspace slots (get_workspace): 0 GEMM partials and tickets, 1 int8
 // quantization staging, 2 the column-major hook's temporary C, 3 transposed
-// bf16 A operands.
-constexpr int kSlotGemm = 0, kSlotQuant = 1, kSlotHookC = 2, kSlotTransA = 3;
+// bf16 A operands, 4 bf16 copies of fp32 operands.
+constexpr int kSlotGemm = 0, kSlotQuant = 1, kSlotHookC = 2, kSlotTransA = 3, kSlotBf16 = 4;
 
 }  // namespace dnnopt_hip

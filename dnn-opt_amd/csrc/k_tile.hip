@@ -533,7 +533,17 @@ __device__ __forceinline__ int bseg_swz(int k) { return (k & 3) | (((k >> 3) & 1
 // sub-tile (the WM x WN output waves are replicated KW times); their sums
 // are added in ascending order through LDS after the loop.  Fewer, larger
 // per-wave sub-tiles read fewer operand bytes from LDS per MFMA.
-template <int MT, int NT, int WM, int WN, int D, int MODE, int TB = 0, int KB0 = 0, int KW = 1>
+//
+// RAW = 1 (fp32 operands): elements stay unrounded in the register ring and
+// are rounded when they are written to LDS.  Rounded on arrival (RAW = 0),
+// every iteration waits for the loads it has just issued, but the ring takes
+// half the registers.  Measured on 10 shapes, M = 16..256 (MI355X, RAW 0 ->
+// 1, geometric mean): 128 x 96 1.18x (64-k blocks) and 1.14x (128-k), 256 x
+// 96 1.19x, 64 x 128 on 8 waves 1.13x, 64 x 64 1.06x; but 32 x 64 with 256-k
+// blocks 0.88x, 32 x 128 0.94x, 64 x 128 on 4 waves 0.89x, and 32 x 64 with
+// 128-k blocks 1.04-1.16x while every workgroup has a CU to itself, 0.86-0.98x
+// beyond that.
+template <int MT, int NT, int WM, int WN, int D, int MODE, int TB = 0, int KB0 = 0, int KW = 1, int RAW = 0>
 __global__ __launch_bounds__(WM* WN * KW * 64) void dnnopt_tile_bf16_lds(TileArgs p) {
     static_assert(!TB || MODE == kTileBF16, "B stored N x K needs bf16 storage");
     using S = TileShape<MT, NT, WM, WN, 1>;
@@ -578,16 +588,16 @@ __global__ __launch_bounds__(WM* WN * KW * 64) void dnnopt_tile_bf16_lds(TileArg
     const int b_lo = (int)(((long long)nblk * blockIdx.z) / p.splits);
     const int b_hi = (int)(((long long)nblk * (blockIdx.z + 1)) / p.splits);
 
-    constexpr int ES = MODE == kTileBF16 ? 2 : 4;
-    const char* abase = static_cast<const char*>(p.A) + (size_t)m0 * p.lda * ES;
-    const char* bbase = static_cast<const char*>(p.B) + (TB ? (size_t)n0 * p.ldb : (size_t)n0) * ES;
+    constexpr int ESA = MODE == kTileF2B ? 4 : 2, ESB = MODE == kTileBF16 ? 2 : 4;
+    const char* abase = static_cast<const char*>(p.A) + (size_t)m0 * p.lda * ESA;
+    const char* bbase = static_cast<const char*>(p.B) + (TB ? (size_t)n0 * p.ldb : (size_t)n0) * ESB;
     // Ranges end at the last element of each operand, rounded up to a whole
     // dword: the range check of a dword load drops a dword that extends past
     // the range, and the last element may share its dword with the next.
     const __amdgpu_buffer_rsrc_t ra =
-        make_rsrc(abase, clamp_rec((((size_t)(p.M - 1 - m0) * p.lda + p.K) * ES + 3) & ~(size_t)3));
+        make_rsrc(abase, clamp_rec((((size_t)(p.M - 1 - m0) * p.lda + p.K) * ESA + 3) & ~(size_t)3));
     const size_t b_last = TB ? (size_t)(p.N - 1 - n0) * p.ldb + p.K : (size_t)(p.K - 1) * p.ldb + (p.N - n0);
-    const __amdgpu_buffer_rsrc_t rb = make_rsrc(bbase, clamp_rec((b_last * ES + 3) & ~(size_t)3));
+    const __amdgpu_buffer_rsrc_t rb = make_rsrc(bbase, clamp_rec((b_last * ESB + 3) & ~(size_t)3));
 
     // Per-thread offsets that do not change from block to block are computed
     // once: global element offsets of this thread's A chunks and B rows (an
@@ -600,7 +610,7 @@ __global__ __launch_bounds__(WM* WN * KW * 64) void dnnopt_tile_bf16_lds(TileArg
     for (int i = 0; i < AU; ++i) {
         const int idx = t + i * NTH, row = idx / CPR, c = idx % CPR;
         const bool ok = (ACH % NTH == 0 || idx < ACH) && m0 + row < p.M;
-        a_off[i] = ok ? ((uint32_t)row * p.lda + 8 * c) * ES : kOobOffset;
+        a_off[i] = ok ? ((uint32_t)row * p.lda + 8 * c) * ESA : kOobOffset;
         a_lds[i] = row * ROWB + swz_a(row, c) * 16;
         a_c[i] = 8 * c;
     }
@@ -609,14 +619,14 @@ __global__ __launch_bounds__(WM* WN * KW * 64) void dnnopt_tile_bf16_lds(TileArg
         if constexpr (TB) {
             const int idx = t + i * NTH, row = idx / CPR, c = idx % CPR;
             const bool ok = (BUN % NTH == 0 || idx < BUN) && n0 + row < p.N;
-            b_off[i] = ok ? ((uint32_t)row * p.ldb + 8 * c) * ES : kOobOffset;
+            b_off[i] = ok ? ((uint32_t)row * p.ldb + 8 * c) * ESB : kOobOffset;
             b_lds[i] = row * ROWB + swz_a(row, c) * 16;
             b_c[i] = 8 * c;
         } else {
             const int u = t + i * NTH, cg = u % (BN / 8), kr = u / (BN / 8);
             const bool ok = BUN % NTH == 0 || u < BUN;
             b_c[i] = 0;
-            b_off[i] = ok ? ((uint32_t)kr * p.ldb + 8 * cg) * ES : kOobOffset;
+            b_off[i] = ok ? ((uint32_t)kr * p.ldb + 8 * cg) * ESB : kOobOffset;
             b_lds[i] = ok ? kr * BROW + cg * 16 : -1;
         }
     }
@@ -626,31 +636,31 @@ __global__ __launch_bounds__(WM* WN * KW * 64) void dnnopt_tile_bf16_lds(TileArg
     // range by up to D - 1 blocks; those re-read the last block (never used),
     // so every load is unconditional and the compiler waits for exactly the
     // loads each LDS store needs.
-    u32x4 sa[D][AU], sb[D][BU];
+    constexpr int LA = ESA / 2, LB = ESB / 2;                  // 16-byte loads per chunk
+    constexpr int RA = RAW ? LA : 1, RB = RAW ? LB : 1;        // 16-byte pieces per chunk in the ring
+    u32x4 sa[D][AU][RA], sb[D][BU][RB];
+    auto chunk = [](const auto& v) {
+        if constexpr (sizeof v == sizeof(u32x4)) return v[0];
+        else return pack_bf16x8(v[0], v[1]);
+    };
+    auto fetch = [](auto& v, __amdgpu_buffer_rsrc_t r, uint32_t off, auto loads) {
+        constexpr int L = decltype(loads)::value;
+        if constexpr (L == 2 && !RAW) {
+            const u32x4 lo = buf_load_x4(r, off), hi = buf_load_x4(r, off + 16u);
+            v[0] = pack_bf16x8(lo, hi);
+        } else {
+#pragma unroll
+            for (int q = 0; q < L; ++q) v[q] = buf_load_x4(r, off + 16u * q);
+        }
+    };
     auto load_stage = [&](int blk, int slot) {
         const int bc = blk < b_hi ? blk : b_hi - 1;
-        const uint32_t ka = (uint32_t)bc * BK * ES;
-        const uint32_t kb = TB ? ka : (uint32_t)bc * BK * p.ldb * ES;
+        const uint32_t ka = (uint32_t)bc * BK * ESA;
+        const uint32_t kb = TB ? (uint32_t)bc * BK * ESB : (uint32_t)bc * BK * p.ldb * ESB;
 #pragma unroll
-        for (int i = 0; i < AU; ++i) {
-            if constexpr (MODE == kTileBF16) {
-                sa[slot][i] = buf_load_x4(ra, a_off[i] + ka);
-            } else {
-                const u32x4 lo = buf_load_x4(ra, a_off[i] + ka);
-                const u32x4 hi = buf_load_x4(ra, a_off[i] + ka + 16u);
-                sa[slot][i] = pack_bf16x8(lo, hi);
-            }
-        }
+        for (int i = 0; i < AU; ++i) fetch(sa[slot][i], ra, a_off[i] + ka, std::integral_constant<int, LA>{});
 #pragma unroll
-        for (int i = 0; i < BU; ++i) {
-            if constexpr (MODE == kTileBF16) {
-                sb[slot][i] = buf_load_x4(rb, b_off[i] + kb);
-            } else {
-                const u32x4 lo = buf_load_x4(rb, b_off[i] + kb);
-                const u32x4 hi = buf_load_x4(rb, b_off[i] + kb + 16u);
-                sb[slot][i] = pack_bf16x8(lo, hi);
-            }
-        }
+        for (int i = 0; i < BU; ++i) fetch(sb[slot][i], rb, b_off[i] + kb, std::integral_constant<int, LB>{});
     };
     auto write_stage = [&](int slot, int buf, int blk) {
         char* As = lds + buf * STAGE;
@@ -673,11 +683,11 @@ __global__ __launch_bounds__(WM* WN * KW * 64) void dnnopt_tile_bf16_lds(TileArg
 #pragma unroll
             for (int i = 0; i < AU; ++i)
                 if (ACH % NTH == 0 || t + i * NTH < ACH)
-                    *reinterpret_cast<u32x4*>(As + a_lds[i]) = keep_k(sa[slot][i], kv - a_c[i]);
+                    *reinterpret_cast<u32x4*>(As + a_lds[i]) = keep_k(chunk(sa[slot][i]), kv - a_c[i]);
 #pragma unroll
             for (int i = 0; i < BU; ++i) {
                 if (BUN % NTH != 0 && t + i * NTH >= BUN) continue;
-                *reinterpret_cast<u32x4*>(Bs + b_lds[i]) = TB ? keep_k(sb[slot][i], kv - b_c[i]) : sb[slot][i];
+                *reinterpret_cast<u32x4*>(Bs + b_lds[i]) = TB ? keep_k(chunk(sb[slot][i]), kv - b_c[i]) : chunk(sb[slot][i]);
             }
             // Keeps the masked stores in this branch: merged with the plain
             // path they would become per-element selects on every block.
@@ -686,11 +696,11 @@ __global__ __launch_bounds__(WM* WN * KW * 64) void dnnopt_tile_bf16_lds(TileArg
         }
 #pragma unroll
         for (int i = 0; i < AU; ++i)
-            if (ACH % NTH == 0 || t + i * NTH < ACH) *reinterpret_cast<u32x4*>(As + a_lds[i]) = sa[slot][i];
+            if (ACH % NTH == 0 || t + i * NTH < ACH) *reinterpret_cast<u32x4*>(As + a_lds[i]) = chunk(sa[slot][i]);
 #pragma unroll
         for (int i = 0; i < BU; ++i) {
             if (BUN % NTH != 0 && t + i * NTH >= BUN) continue;
-            *reinterpret_cast<u32x4*>(Bs + b_lds[i]) = sb[slot][i];
+            *reinterpret_cast<u32x4*>(Bs + b_lds[i]) = chunk(sb[slot][i]);
         }
     };
 
@@ -1392,19 +1402,29 @@ TileConfig tile_config(int idx) { return kTileConfigs[idx]; }
         hipLaunchKernelGGL((dnnopt_tile_f32_dma<MT, NT, WM, WN, NS, 1>), grid, blk, 0, s, a);               \
         break;
 
-#define DNNOPT_TILE_LDS_CASE(IDX, MT, NT, WM, WN, D, KB, KW)                                              \
+#define DNNOPT_TILE_LDS_CASE(IDX, MT, NT, WM, WN, D, KB, KW, RAW)                                            \
     case IDX:                                                                                              \
         if (mode == kTileBF16 && tb) hipLaunchKernelGGL((dnnopt_tile_bf16_lds<MT, NT, WM, WN, D, kTileBF16, 1, KB, KW>), grid, blk, 0, s, a); \
         else if (mode == kTileBF16) hipLaunchKernelGGL((dnnopt_tile_bf16_lds<MT, NT, WM, WN, D, kTileBF16, 0, KB, KW>), grid, blk, 0, s, a); \
-        else if (mode == kTileF2B) hipLaunchKernelGGL((dnnopt_tile_bf16_lds<MT, NT, WM, WN, D, kTileF2B, 0, KB, KW>), grid, blk, 0, s, a); \
+        else if (mode == kTileF2B) hipLaunchKernelGGL((dnnopt_tile_bf16_lds<MT, NT, WM, WN, D, kTileF2B, 0, KB, KW, RAW>), grid, blk, 0, s, a); \
         else return hipErrorInvalidValue;                                                                  \
         break;
+
+// A bf16, B fp32 (kTileA16).  A third block in the register ring measured 1%
+// slower on both (256 x 96: 87.4 vs 88.1 us at 512 x 11008 x 4096).
+static hipError_t launch_tile_a16(int cfg_idx, dim3 grid, const TileArgs& a, hipStream_t s) {
+    if (cfg_idx == 20) hipLaunchKernelGGL((dnnopt_tile_bf16_lds<2, 3, 4, 2, 2, kTileA16, 0, 128, 1, 1>), grid, dim3(512), 0, s, a);
+    else if (cfg_idx == kTileF2BTall) hipLaunchKernelGGL((dnnopt_tile_bf16_lds<4, 3, 4, 2, 2, kTileA16, 0, 64, 1, 1>), grid, dim3(512), 0, s, a);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
 
 hipError_t launch_tile(int mode, int cfg_idx, int ta, int tb, int al, dim3 grid, const TileArgs& a, hipStream_t s) {
     // Transposed operands: fp32 both, bf16 storage B only (stored N x K).
     if (mode != kTileF32 && (ta || (tb && mode != kTileBF16))) return hipErrorInvalidValue;
     if (cfg_idx == kTileKOuter) return mode == kTileF32 && ta && !tb ? launch_kouter_f32(grid, a, s) : hipErrorInvalidValue;
     if (cfg_idx < 0 || cfg_idx >= tile_config_count()) return hipErrorInvalidValue;
+    if (mode == kTileA16) return launch_tile_a16(cfg_idx, grid, a, s);
     if (tile_pp(cfg_idx)) {
         if (mode != kTileBF16 || !al) return hipErrorInvalidValue;
         PPArgs q{};
@@ -1425,6 +1445,12 @@ hipError_t launch_tile(int mode, int cfg_idx, int ta, int tb, int al, dim3 grid,
         q.tiles_m = a.tiles_m;
         return launch_pp(0, cfg_idx - kTilePPFirst, tb, 0, grid, q, s);
     }
+    if (cfg_idx == 19 && mode == kTileF2B && (long long)grid.x * grid.z <= 256 && a.K / 128 / a.splits >= 8) {
+        // a CU to every workgroup and 8 blocks or more each (with fewer, its
+        // longer start costs 3-4%): the raw ring (see dnnopt_tile_bf16_lds)
+        hipLaunchKernelGGL((dnnopt_tile_bf16_lds<2, 1, 1, 4, 3, kTileF2B, 0, 128, 1, 1>), grid, dim3(256), 0, s, a);
+        return hipGetLastError();
+    }
     const TileConfig c = kTileConfigs[cfg_idx];
     const dim3 blk(c.wm * c.wn * c.kw * 64);
     if (cfg_idx >= kTileFirstLds && !al) return hipErrorInvalidValue;
@@ -1434,27 +1460,27 @@ hipError_t launch_tile(int mode, int cfg_idx, int ta, int tb, int al, dim3 grid,
         DNNOPT_TILE_CASE(2, 2, 2, 2, 2, 1)
         DNNOPT_TILE_CASE(3, 2, 2, 2, 2, 2)
         DNNOPT_TILE_CASE(4, 2, 4, 2, 2, 1)
-        DNNOPT_TILE_LDS_CASE(5, 4, 4, 2, 2, 2, 0, 1)
-        DNNOPT_TILE_LDS_CASE(6, 2, 2, 1, 4, 2, 0, 1)
-        DNNOPT_TILE_LDS_CASE(7, 2, 4, 2, 2, 2, 0, 1)
-        DNNOPT_TILE_LDS_CASE(8, 4, 4, 2, 2, 3, 0, 1)
-        DNNOPT_TILE_LDS_CASE(9, 4, 4, 2, 2, 4, 0, 1)
-        DNNOPT_TILE_LDS_CASE(10, 2, 2, 1, 4, 4, 0, 1)
-        DNNOPT_TILE_LDS_CASE(11, 2, 4, 2, 2, 4, 0, 1)
-        DNNOPT_TILE_LDS_CASE(12, 4, 2, 2, 4, 3, 0, 1)
-        DNNOPT_TILE_LDS_CASE(13, 2, 3, 4, 2, 3, 0, 1)
-        DNNOPT_TILE_LDS_CASE(14, 2, 3, 4, 2, 2, 0, 1)
-        DNNOPT_TILE_LDS_CASE(15, 4, 2, 2, 4, 2, 0, 1)
-        DNNOPT_TILE_LDS_CASE(16, 2, 1, 1, 4, 2, 256, 1)
-        DNNOPT_TILE_LDS_CASE(17, 2, 2, 1, 2, 2, 256, 1)
-        DNNOPT_TILE_LDS_CASE(18, 2, 2, 1, 4, 2, 128, 1)
-        DNNOPT_TILE_LDS_CASE(19, 2, 1, 1, 4, 3, 128, 1)
-        DNNOPT_TILE_LDS_CASE(20, 2, 3, 4, 2, 2, 128, 1)
-        DNNOPT_TILE_LDS_CASE(21, 2, 2, 2, 2, 3, 128, 1)
-        DNNOPT_TILE_LDS_CASE(22, 2, 4, 2, 2, 2, 128, 1)
-        DNNOPT_TILE_LDS_CASE(23, 2, 2, 2, 4, 2, 128, 1)
-        DNNOPT_TILE_LDS_CASE(24, 4, 3, 2, 2, 3, 0, 2)
-        DNNOPT_TILE_LDS_CASE(25, 4, 3, 2, 2, 6, 0, 2)
+        DNNOPT_TILE_LDS_CASE(5, 4, 4, 2, 2, 2, 0, 1, 0)
+        DNNOPT_TILE_LDS_CASE(6, 2, 2, 1, 4, 2, 0, 1, 0)
+        DNNOPT_TILE_LDS_CASE(7, 2, 4, 2, 2, 2, 0, 1, 0)
+        DNNOPT_TILE_LDS_CASE(8, 4, 4, 2, 2, 3, 0, 1, 0)
+        DNNOPT_TILE_LDS_CASE(9, 4, 4, 2, 2, 4, 0, 1, 0)
+        DNNOPT_TILE_LDS_CASE(10, 2, 2, 1, 4, 4, 0, 1, 0)
+        DNNOPT_TILE_LDS_CASE(11, 2, 4, 2, 2, 4, 0, 1, 0)
+        DNNOPT_TILE_LDS_CASE(12, 4, 2, 2, 4, 3, 0, 1, 1)
+        DNNOPT_TILE_LDS_CASE(13, 2, 3, 4, 2, 3, 0, 1, 1)
+        DNNOPT_TILE_LDS_CASE(14, 2, 3, 4, 2, 2, 0, 1, 1)
+        DNNOPT_TILE_LDS_CASE(15, 4, 2, 2, 4, 2, 0, 1, 1)
+        DNNOPT_TILE_LDS_CASE(16, 2, 1, 1, 4, 2, 256, 1, 0)
+        DNNOPT_TILE_LDS_CASE(17, 2, 2, 1, 2, 2, 256, 1, 0)
+        DNNOPT_TILE_LDS_CASE(18, 2, 2, 1, 4, 2, 128, 1, 0)
+        DNNOPT_TILE_LDS_CASE(19, 2, 1, 1, 4, 3, 128, 1, 0)
+        DNNOPT_TILE_LDS_CASE(20, 2, 3, 4, 2, 2, 128, 1, 1)
+        DNNOPT_TILE_LDS_CASE(21, 2, 2, 2, 2, 3, 128, 1, 1)
+        DNNOPT_TILE_LDS_CASE(22, 2, 4, 2, 2, 2, 128, 1, 0)
+        DNNOPT_TILE_LDS_CASE(23, 2, 2, 2, 4, 2, 128, 1, 1)
+        DNNOPT_TILE_LDS_CASE(24, 4, 3, 2, 2, 3, 0, 2, 0)
+        DNNOPT_TILE_LDS_CASE(25, 4, 3, 2, 2, 6, 0, 2, 0)
         DNNOPT_TILE_DMA_CASE(26, 2, 3, 4, 2, 3, 64)
         DNNOPT_TILE_DMA_CASE(27, 2, 3, 4, 2, 4, 64)
         DNNOPT_TILE_DMA_CASE(28, 2, 1, 1, 4, 3, 128)
@@ -1466,10 +1492,10 @@ hipError_t launch_tile(int mode, int cfg_idx, int ta, int tb, int al, dim3 grid,
         DNNOPT_TILE_DMA_CASE(34, 4, 4, 4, 2, 3, 64)
         DNNOPT_TILE_CASE(35, 1, 1, 1, 1, 8)
         DNNOPT_TILE_CASE(36, 1, 4, 1, 2, 2)
-        DNNOPT_TILE_LDS_CASE(37, 2, 1, 1, 3, 3, 128, 1)
-        DNNOPT_TILE_LDS_CASE(38, 1, 1, 1, 3, 3, 128, 1)
+        DNNOPT_TILE_LDS_CASE(37, 2, 1, 1, 3, 3, 128, 1, 0)
+        DNNOPT_TILE_LDS_CASE(38, 1, 1, 1, 3, 3, 128, 1, 0)
         DNNOPT_TILE_DMA_CASE(39, 4, 4, 2, 2, 3, 64)
-        DNNOPT_TILE_LDS_CASE(40, 4, 3, 4, 2, 2, 64, 1)
+        DNNOPT_TILE_LDS_CASE(40, 4, 3, 4, 2, 2, 64, 1, 1)
         DNNOPT_TILE_F32DMA_CASE(41, 2, 4, 2, 2, 3)
         DNNOPT_TILE_F32DMA_CASE(42, 4, 4, 2, 2, 3)
         DNNOPT_TILE_F32DMA_CASE(43, 1, 4, 4, 1, 3)

@@ -180,6 +180,7 @@ enum TileMode {
     kTileF32 = 0,
     kTileBF16 = 1,
     kTileF2B = 2,
+    kTileA16 = 3,  // A bf16 storage, B fp32 rounded to bf16 (LDS-staged tiles)
 };
 
 struct TileArgs {
@@ -382,6 +383,13 @@ hipError_t launch_s8_reduce(const int32_t* part, int splits, int tiles_n, int ti
 hipError_t launch_splitk_reduce(const float* part, int splits, int tiles_n, int tiles_m, int bm,
                                 int bn, int M, int N, float alpha, float beta, float* C, int ldc,
                                 const float* bias, hipStream_t s);
+
+// bf16 copies of fp32 operands (nearest even, the reference formula): A (M x
+// K) into dA (row stride ldda) and, unless dB is null, B (K x N) into dB (dK
+// >= K rows of stride lddb); the padding columns and rows of the copies are zero.  ldda, lddb
+// multiples of 8; 16 lda, 16 ldb below 2^31.
+hipError_t launch_bf16_copy(const float* A, int lda, const float* B, int ldb, int M, int N, int K, uint16_t* dA,
+                            int ldda, uint16_t* dB, int lddb, int dK, hipStream_t s);
 
 // Column-major helpers of the oneDNN-hook entry points.  C(i, j) is at
 // C[j * ldc + i]; ldc < M means overlapping columns (see k_colmajor.hip).

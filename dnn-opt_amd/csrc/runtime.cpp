@@ -139,6 +139,48 @@ hipStream_t thread_stream(int* status) {
     return s;
 }
 
+void* optional_workspace(hipStream_t s, size_t bytes, int slot) {
+    int dev = 0;
+    if (bytes > kOptionalBytes || hipGetDevice(&dev) != hipSuccess) return nullptr;
+    // A graph would keep the address, which a later, larger call may free.
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    Scratch* w = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(g_ws_mu);
+        w = &g_ws[{{dev, slot}, s}];
+    }
+    if (w->ptr && w->cap >= bytes) return w->ptr;
+    // Another stream's capture, on any thread, does not forbid this one's
+    // allocation (and must not be ended by it).
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    hipError_t e = hipSuccess;
+    if (w->ptr) {
+        // Launches already queued on this stream may still use the old buffer.
+        e = hipStreamSynchronize(s);
+        if (e == hipSuccess) {
+            (void)hipFree(w->ptr);
+            w->ptr = nullptr;
+            w->cap = 0;
+        }
+    }
+    if (e == hipSuccess) {
+        e = hipMalloc(&w->ptr, bytes);
+        if (e == hipSuccess) w->cap = bytes;
+        else w->ptr = nullptr;
+    }
+    if (e != hipSuccess) (void)hipGetLastError();
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return e == hipSuccess ? w->ptr : nullptr;
+}
+
 int get_workspace(hipStream_t s, size_t part_bytes, void** part, unsigned** tickets, int slot) {
     if (visible_devices() == 0) return DNNOPT_ERR_NO_DEVICE;
     int dev = 0;

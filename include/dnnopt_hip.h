@@ -244,6 +244,10 @@ int dnnopt_hip_plan_sgemm(int transA, int transB, int M, int N, int K,
  * operand with 32-bit offsets are only chosen when its strides allow. */
 int dnnopt_hip_plan_sgemm_ex(int transA, int transB, int M, int N, int K,
                              int lda, int ldb, int ldc, dnnopt_plan* out);
+/* fp32_inputs = 1: the launch that rounds the operands while staging them.  A
+ * call with many rows may instead round A, or both operands, once into library
+ * workspace and run the tiles on the copies (never while its stream is being
+ * captured). */
 int dnnopt_hip_plan_gemm_bf16(int fp32_inputs, int M, int N, int K,
                               dnnopt_plan* out);
 int dnnopt_hip_plan_gemm_bf16_ex(int transA, int transB, int M, int N, int K,

@@ -1,0 +1,108 @@
+"""The fp32-input bf16 GEMM on operands rounded ahead into workspace: A alone,
+or both (many rows), against the fp64 product of the bf16-rounded operands;
+ragged sizes, padded strides with NaN in the padding, beta, rounding ties and
+special values; calls under graph capture, which keep to the direct tiles."""
+
+import numpy as np
+import pytest
+
+import _util as u
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+def dev_copy(x, device):
+    return torch.from_numpy(np.ascontiguousarray(x)).to(device)
+
+
+def host(t):
+    torch.cuda.synchronize()
+    return t.cpu().numpy()
+
+
+def stream():
+    return torch.cuda.current_stream().cuda_stream
+
+
+# The models round A alone (128 x 96 tiles, 256 x 96 tiles, a k-split) or both
+# operands (from about 700 rows) on these; the last two keep the direct tiles.
+SHAPES = [(200, 9000, 1000, 0, 1.0, 0.0), (380, 10007, 777, 3, 0.5, 1.0), (513, 2500, 1501, 1, -2.0, 0.25),
+          (1024, 4100, 520, 2, 1.0, 0.0), (1030, 2049, 1003, 5, 1.0, 1.0), (300, 500, 129, 1, 1.0, 0.0),
+          (65, 130, 64, 0, 1.0, 1.0)]
+
+
+@pytest.mark.parametrize("M,N,K,pad,alpha,beta", SHAPES)
+def test_against_rounded_operands(lib, orc, dev, M, N, K, pad, alpha, beta):
+    A, B = u.normal(orc, M * K, 1).reshape(M, K), u.normal(orc, K * N, 2, 0, 0.02).reshape(K, N)
+    sa, sb = np.full((M, K + pad), np.nan, np.float32), np.full((K, N + pad), np.nan, np.float32)
+    sa[:, :K], sb[:, :N] = A, B
+    C0 = u.uniform(orc, M * N, 3).reshape(M, N)
+    want, scale = u.exact(u.bf16_value(u.bf16_bits(orc, A)), u.bf16_value(u.bf16_bits(orc, B)), alpha, beta, C0)
+    dA, dB = dev_copy(sa, dev), dev_copy(sb, dev)
+    got = []
+    for _ in range(2):
+        dC = dev_copy(C0 if beta else np.full_like(C0, np.nan), dev)
+        lib.gemm_bf16_f32in(M, N, K, alpha, dA, K + pad, dB, N + pad, beta, dC, N, stream=stream())
+        got.append(host(dC))
+    u.assert_fp32_close(got[0], want, scale, K, f"{M}x{N}x{K}")
+    u.assert_bits_equal(got[0], got[1], "repeated call")
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 9000, 1024), (1024, 4096, 512)])
+def test_rounding_and_special_values(lib, orc, dev, M, N, K):
+    """One nonzero of A per row (1.0): C's row is a row of B, rounded.  Ties,
+    subnormals, infinities and NaNs of B come out as the rounding formula
+    leaves them."""
+    rng = np.random.default_rng(5)
+    B = rng.integers(0, 1 << 32, (K, N), dtype=np.uint64).astype(np.uint32)
+    B[:, ::3] = (B[:, ::3] & 0xFFFF0000) | 0x8000  # ties
+    B &= 0xBFFFFFFF  # finite (exponents below 2^0) ...
+    B[:, 7] = 0x7F800000  # ... but for a column each of inf and NaN
+    B[:, 11] = 0x7FC00000
+    A = np.zeros((M, K), np.float32)
+    pick = rng.integers(0, K, M)
+    A[np.arange(M), pick] = 1.0
+    dC = torch.full((M, N), float("nan"), device=dev)
+    lib.gemm_bf16_f32in(M, N, K, 1.0, dev_copy(A, dev), K, dev_copy(B.view(np.float32), dev), N, 0.0, dC, N, stream=stream())
+    got = host(dC)
+    want = u.bf16_value(u.bf16_bits(orc, np.ascontiguousarray(B.view(np.float32)[pick])))
+    cols = np.ones(N, bool)
+    cols[[7, 11]] = False  # 0 * inf and 0 * NaN of the other rows make NaN there
+    # the matrix cores flush no bf16 operand, but a product below the fp32 normals may differ
+    normal = np.abs(want[:, cols]) >= 2.0 ** -126
+    assert np.array_equal(got[:, cols][normal], want[:, cols][normal])
+    assert np.isnan(got[:, [7, 11]]).all()
+
+
+def test_under_graph_capture(lib, orc, dev):
+    """A captured call rounds while staging (a graph must not keep the address
+    of workspace that a later call may free), whether or not its stream has
+    workspace already; replays between eager calls, one of which grows the
+    workspace, stay within the bound."""
+    M, N, K = 512, 8192, 512
+    A, B = u.normal(orc, M * K, 1).reshape(M, K), u.normal(orc, K * N, 2, 0, 0.02).reshape(K, N)
+    want, scale = u.exact(u.bf16_value(u.bf16_bits(orc, A)), u.bf16_value(u.bf16_bits(orc, B)))
+    dA, dB = dev_copy(A, dev), dev_copy(B, dev)
+    for warm in (False, True):
+        s = torch.cuda.Stream()
+        dC, dE = torch.full((M, N), float("nan"), device=dev), torch.full((M, N), float("nan"), device=dev)
+        torch.cuda.synchronize()
+        if warm:
+            lib.gemm_bf16_f32in(M, N, K, 1.0, dA, K, dB, N, 0.0, dE, N, stream=s.cuda_stream)
+            torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            lib.gemm_bf16_f32in(M, N, K, 1.0, dA, K, dB, N, 0.0, dC, N, stream=s.cuda_stream)
+        for rep in range(3):
+            dC.fill_(float("nan"))
+            torch.cuda.synchronize()
+            g.replay()
+            u.assert_fp32_close(host(dC), want, scale, K, f"replay {rep}, warm={warm}")
+            lib.gemm_bf16_f32in(M, N, K, 1.0, dA, K, dB, N, 0.0, dE, N, stream=s.cuda_stream)
+            u.assert_fp32_close(host(dE), want, scale, K, f"eager {rep}, warm={warm}")
+            if rep == 0:  # a larger call on the same stream
+                big = torch.zeros((2048, 4096), device=dev)
+                lib.gemm_bf16_f32in(2048, 4096, 2048, 1.0, torch.zeros((2048, 2048), device=dev), 2048,
+                                    torch.zeros((2048, 4096), device=dev), 4096, 0.0, big, 4096, stream=s.cuda_stream)
+                torch.cuda.synchronize()
