@@ -361,6 +361,17 @@ static int gemm_bf16_common(int fp32_inputs, int M, int N, int K, float alpha, c
         return run_skinny(L, A, lda, 1, B, ldb, C, ldc, M, N, K, alpha, beta, s);
     Bf16Copies cp{};
     if (fp32_inputs && plan_bf16_copies(L, M, N, K, lda, ldb, ldc, &cp)) {
+        // A later call of this size may be captured, and then takes the tiles
+        // below: their split-k workspace is grown now, as it would be without
+        // the copies.
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (L.grid.z > 1 && hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
+            void* part = nullptr;
+            unsigned* tickets = nullptr;
+            st = get_workspace(s, L.part_bytes, &part, &tickets);
+            if (st != DNNOPT_OK) return st;
+        }
+        (void)hipGetLastError();
         // Operands rounded once into workspace (k padded with zeros to a
         // multiple of 8) ahead of the tiles.  Without the workspace (under
         // capture, or when memory is short) the tiles below round both while

@@ -106,3 +106,28 @@ def test_under_graph_capture(lib, orc, dev):
                 lib.gemm_bf16_f32in(2048, 4096, 2048, 1.0, torch.zeros((2048, 2048), device=dev), 2048,
                                     torch.zeros((2048, 4096), device=dev), 4096, 0.0, big, 4096, stream=s.cuda_stream)
                 torch.cuda.synchronize()
+
+
+def test_captured_after_a_warm_call(lib, orc, dev):
+    """Eager calls take the rounded copies, a captured one the split tiles: its
+    split-k workspace is there after the warm-up call on the same stream."""
+    M, N, K = 284, 2304, 3904
+    assert lib.plan_bf16(M, N, K, fp32_inputs=1)["splits"] > 1
+    A, B = u.normal(orc, M * K, 1).reshape(M, K), u.normal(orc, K * N, 2, 0, 0.02).reshape(K, N)
+    want, scale = u.exact(u.bf16_value(u.bf16_bits(orc, A)), u.bf16_value(u.bf16_bits(orc, B)))
+    dA, dB = dev_copy(A, dev), dev_copy(B, dev)
+    dC = torch.full((M, N), float("nan"), device=dev)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    call = lambda: lib.gemm_bf16_f32in(M, N, K, 1.0, dA, K, dB, N, 0.0, dC, N, stream=s.cuda_stream)
+    call()
+    torch.cuda.synchronize()
+    u.assert_fp32_close(host(dC), want, scale, K, "warm-up")
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        call()
+    for rep in range(3):
+        dC.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        u.assert_fp32_close(host(dC), want, scale, K, f"replay {rep}")
