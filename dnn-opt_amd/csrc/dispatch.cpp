@@ -462,6 +462,21 @@ static const WgFit kS8Fit[] = {
 static const WgModel kBf16PPModel{kBf16PPFit, (int)(sizeof kBf16PPFit / sizeof kBf16PPFit[0]), 2, 3.007, 2.543, 0.152, 0.439};
 static const WgModel kS8Model{kS8Fit, (int)(sizeof kS8Fit / sizeof kS8Fit[0]), 1, 1.5, 2.801, 0.198, 0.381};
 
+// fp32 tiles whose waves split k (k_wavek.hip): about 100 shapes per layout of
+// B (M = 12..2048, N = 64..4096, K = 128..4096; 7 tiles, 1 to 4 splits): median
+// error 2.5%, 90% within 7%.  Only 32 x 48 with B stored N x K leaves LDS for
+// a second workgroup.
+static const WgFit kWavekTbFit[] = {
+    {64, 1, 2.935, 0.564, 0.0}, {58, 1, 4.094, 1.156, 0.0}, {59, 1, 4.541, 1.034, 0.0}, {60, 1, 3.134, 0.796, 0.0},
+    {61, 1, 2.813, 0.617, 0.0}, {62, 1, 2.882, 0.563, 0.0}, {63, 2, 2.397, 0.431, 0.904},
+};
+static const WgFit kWavekFit[] = {
+    {64, 1, 2.603, 0.612, 0.0}, {58, 1, 3.693, 1.201, 0.0}, {59, 1, 4.108, 1.067, 0.0}, {60, 1, 2.776, 0.851, 0.0},
+    {61, 1, 2.536, 0.672, 0.0}, {62, 1, 2.632, 0.577, 0.0}, {63, 1, 2.118, 0.491, 0.0},
+};
+static const WgModel kWavekTbModel{kWavekTbFit, 7, 4, 1.382, 2.364, 0.161, 0.0};
+static const WgModel kWavekModel{kWavekFit, 7, 4, 1.802, 2.309, 0.194, 0.0};
+
 static double wg_cost(const WgModel& md, const WgFit& f, int bm, int bn, int kb, long long s, int M, int N, int K,
                       long long cus) {
     const long long tiles = ceil_div(M, bm) * ceil_div(N, bn), blocks = ceil_div(ceil_div(K, kb), s);
@@ -575,7 +590,7 @@ static TilePick pick_f32_tile(int tb, int M, int N, int K, int def_cfg) {
 // 32-column wave tiles need B stored N x K.
 static bool f32_dma_fits(int cfg, int transA, int transB, int M, int K, int lda, int ldb) {
     (void)M;
-    if (transA || (!transB && cfg >= kTileF32DmaTbFirst)) return false;
+    if (transA || (!transB && cfg >= kTileF32DmaTbFirst && cfg <= kTileF32DmaLast)) return false;
     const TileConfig c = tile_config(cfg);
     const long long bm = c.wm * c.mt * 16, bn = c.wn * c.nt * 16;
     return (bm * lda + K) * 4 < 0x7FFFFFFFll &&
@@ -729,11 +744,44 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
             // the register tiles' model, then the LDS-DMA tiles where their
             // model puts them 10% ahead of that choice
             const TilePick pick = pick_f32_tile(transB ? 1 : 0, M, N, K, cfg);
+            double us = pick.us;
             cfg = pick.cfg;
             model_splits = pick.s;
             if (dma.s > 0 && pick.us > 0.0 && dma.us < 0.9 * pick.us) {
                 cfg = dma.cfg;
                 model_splits = dma.s;
+                us = dma.us;
+            }
+            // k_wavek.hip's tiles where their model puts them 10% ahead of
+            // that choice (MI355X, us: 384 x 3072 x 768 23.9 -> 20.6 (B N x
+            // K, 96 x 48) and 27.5 -> 21.1 (K x N), 384 x 768 x 768 11.1 ->
+            // 9.0, 926 x 561 x 907 20.5 -> 14.1, 134 x 2354 x 393 11.1 ->
+            // 7.8).  Kept from them: up to 32 rows (the 16-row tiles, 16 x
+            // 3712 x 384 4.6 vs 6.3), and with a K x N B up to 128 rows and
+            // from K = 4096, where existing plans are relied on (128 x 3072 x
+            // 768 is to be split, 128 and 512 x 4096 x 4096 on 64 x 128 tiles;
+            // 128 x 4096 x 4096 would take 44 us instead of 55 on 64 x 32).
+            // Rows that are not whole 16-byte chunks slow the copies, which
+            // the model does not price: B N x K then keeps the other tiles
+            // (801 x 3414 x 175 16.6 vs 26.5), as it does below four blocks of
+            // k (1600 x 256 x 192 5.2 vs 6.0); B K x N takes the tiles up to
+            // 64 x 32 (1314 x 203 x 631 19.3 -> 9.4, 920 x 258 x 1178 18.0 ->
+            // 13.3), not the larger (1465 x 3567 x 706 86.6 vs 110.7).
+            const bool whole = ((lda | ldb) & 3) == 0;
+            if (us > 0.0 && M > (transB ? 32 : 128) && (transB ? whole && K >= 256 : K < 4096) &&
+                128LL * ldc * 4 < 0x7FFFFFFFll) {
+                const TilePick wk = best_wg_tile(transB ? kWavekTbModel : kWavekModel, M, N, K,
+                                                 [&](int k, int* bm_, int* bn_, int* kb_) {
+                    const TileConfig t = tile_config(k);
+                    *bm_ = t.mt * 16;
+                    *bn_ = t.nt * 16;
+                    *kb_ = t.kblk;
+                    return (whole || *bm_ * *bn_ <= 64 * 32) && f32_dma_fits(k, transA, transB, M, K, lda, ldb);
+                });
+                if (wk.s > 0 && wk.us < 0.90 * us) {
+                    cfg = wk.cfg;
+                    model_splits = wk.s;
+                }
             }
         } else if (dma.s > 0) {
             // beyond the fitted range (MFMA-bound): the LDS-DMA tiles
@@ -743,9 +791,11 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
     }
     if (!lds && mode == kTileF32 &&
         ((forced_cfg >= 1 && forced_cfg <= 4) || forced_cfg == kTileF32Few || forced_cfg == kTileF32Few128 ||
-         (tile_f32_dma(forced_cfg) && f32_dma_fits(forced_cfg, transA, transB, M, K, lda, ldb))))
+         ((tile_f32_dma(forced_cfg) || (tile_wavek(forced_cfg) && 128LL * ldc * 4 < 0x7FFFFFFFll)) &&
+          f32_dma_fits(forced_cfg, transA, transB, M, K, lda, ldb))))
         cfg = forced_cfg;
-    const bool f32dma = mode == kTileF32 && tile_f32_dma(cfg);
+    const bool wavek = mode == kTileF32 && tile_wavek(cfg);
+    const bool f32dma = mode == kTileF32 && (tile_f32_dma(cfg) || wavek);
     const TileConfig c = tile_config(cfg);
     const int bm = c.wm * c.mt * 16, bn = c.wn * c.nt * 16;
     const int kb = lds || f32dma ? tile_lds_bk(bm, bn, c.kblk) : (mode == kTileF32 ? 64 : 128);
@@ -803,7 +853,7 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
     // finish a tile adds the others' partials.
     const bool dma_ticket = tunable(kTuneTileTicket) == 1;
     const bool dma = (cfg >= kTileFirstDma && cfg < kTileF32Few) || cfg == kTileBF16Dma4w || tile_pp(cfg);  // LDS-DMA tiles
-    const bool ticket_ok = !lds || (dma_ticket && dma && !tile_pp(cfg));
+    const bool ticket_ok = (!lds && !wavek) || (dma_ticket && dma && !tile_pp(cfg));
     // Split sums: fp32 tiles (register and LDS-DMA) let the tile's
     // last-arriving workgroup add up to 8 splits' partials (one kernel; its
     // threads read the partial block in 16-byte pieces, 8 in flight each),

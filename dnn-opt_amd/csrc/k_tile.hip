@@ -1359,6 +1359,14 @@ static const TileConfig kTileConfigs[] = {
     {4, 4, 2, 4, 1, 2, 64},   // 55: 128 x 256
     {4, 3, 2, 4, 1, 2, 64},   // 56: 128 x 192
     {8, 1, 2, 4, 1, 2, 64},   // 57: 256 x 64
+    // fp32, four waves splitting k (k_wavek.hip): {MT, NT, 1, 1, 4, blocks ahead, k per block}
+    {6, 3, 1, 1, 4, 3, 64},   // 58: 96 x 48
+    {4, 4, 1, 1, 4, 3, 64},   // 59: 64 x 64
+    {4, 3, 1, 1, 4, 3, 64},   // 60: 64 x 48
+    {3, 3, 1, 1, 4, 3, 64},   // 61: 48 x 48
+    {4, 2, 1, 1, 4, 3, 64},   // 62: 64 x 32
+    {2, 3, 1, 1, 4, 3, 64},   // 63: 32 x 48
+    {2, 4, 1, 1, 4, 3, 64},   // 64: 32 x 64
 };
 
 int tile_config_count() { return (int)(sizeof(kTileConfigs) / sizeof(kTileConfigs[0])); }
@@ -1424,6 +1432,8 @@ hipError_t launch_tile(int mode, int cfg_idx, int ta, int tb, int al, dim3 grid,
     if (mode != kTileF32 && (ta || (tb && mode != kTileBF16))) return hipErrorInvalidValue;
     if (cfg_idx == kTileKOuter) return mode == kTileF32 && ta && !tb ? launch_kouter_f32(grid, a, s) : hipErrorInvalidValue;
     if (cfg_idx < 0 || cfg_idx >= tile_config_count()) return hipErrorInvalidValue;
+    if (tile_wavek(cfg_idx))
+        return mode == kTileF32 && !ta ? launch_tile_f32_wavek(cfg_idx - kTileWavekFirst, tb, grid, a, s) : hipErrorInvalidValue;
     if (mode == kTileA16) return launch_tile_a16(cfg_idx, grid, a, s);
     if (tile_pp(cfg_idx)) {
         if (mode != kTileBF16 || !al) return hipErrorInvalidValue;

@@ -262,6 +262,10 @@ constexpr int kTileF32DmaFirst = 41, kTileF32DmaTbFirst = 48, kTileF32DmaLast = 
 // kTilePPFirst + i is launch_pp's i.  K a multiple of 8, 256 ldc 4 < 2^31.
 constexpr int kTilePPFirst = 51, kTilePPLast = 57;
 constexpr bool tile_pp(int cfg) { return cfg >= kTilePPFirst && cfg <= kTilePPLast; }
+// fp32, four waves that split k (k_wavek.hip; A stored M x K): configuration
+// kTileWavekFirst + i is launch_tile_f32_wavek's i.
+constexpr int kTileWavekFirst = 58, kTileWavekLast = 64;
+constexpr bool tile_wavek(int cfg) { return cfg >= kTileWavekFirst && cfg <= kTileWavekLast; }
 constexpr bool tile_f32_dma(int cfg) { return cfg >= kTileF32DmaFirst && cfg <= kTileF32DmaLast; }
 // k per LDS block of an LDS-staged configuration: its kblk (or
 // DNNOPT_LDS_KB) when both stages fit in 128 KiB of LDS, else 64.
@@ -272,7 +276,8 @@ constexpr int tile_lds_bk(int bm, int bn, int kblk) {
 // fp32, A stored K x M and B stored K x N, 32 < M, N <= 64, a long k; one
 // 64 x 64 partial tile per k-split (grid = (1, 1, splits), 256 threads),
 // always followed by the split-K reduce kernel.
-constexpr int kTileKOuter = 64;
+constexpr int kTileKOuter = 1000;
+hipError_t launch_tile_f32_wavek(int cfg, int tb, dim3 grid, const TileArgs& a, hipStream_t s);
 hipError_t launch_kouter_f32(dim3 grid, const TileArgs& a, hipStream_t s);
 // transA: fp32 only; transB: fp32, or bf16 storage with B stored N x K.
 // aligned: all k-contiguous rows (A; B stored N x K) start on 4-byte
