@@ -121,6 +121,9 @@ enum Tunable {
 };
 int tunable(Tunable t);
 int tunable_default(Tunable t);
+// Counts the changes of any tunable: a plan made under an earlier count is not
+// reused.
+unsigned tunable_epoch();
 
 int plan_skinny(int mode, int M, int N, int K, int ldb, Launch* L);
 // fp32, large M, N <= 64, B small enough to stay in LDS (no transposed A).

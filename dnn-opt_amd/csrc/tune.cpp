@@ -42,6 +42,7 @@ constexpr TuneDef kDefs[kTuneCount] = {
 };
 
 std::atomic<int> g_val[kTuneCount];
+std::atomic<unsigned> g_epoch{0};
 std::once_flag g_init;
 
 void init_table() {
@@ -68,6 +69,8 @@ int tunable(Tunable t) {
     return g_val[t].load(std::memory_order_relaxed);
 }
 
+unsigned tunable_epoch() { return g_epoch.load(std::memory_order_acquire); }
+
 int tunable_default(Tunable t) { return kDefs[t].dflt; }
 
 }  // namespace dnnopt_hip
@@ -77,6 +80,7 @@ extern "C" int dnnopt_hip_set_tunable(int key, int value, int* previous) {
     if (key < 0 || key >= kTuneCount) return DNNOPT_ERR_INVALID_ARG;
     std::call_once(g_init, init_table);
     const int old = g_val[key].exchange(value, std::memory_order_relaxed);
+    if (old != value) g_epoch.fetch_add(1, std::memory_order_release);
     if (previous) *previous = old;
     return DNNOPT_OK;
 }
