@@ -66,10 +66,21 @@ __device__ __forceinline__ f32x4 load4(const float* row, int c, int cols) {
 
 }  // namespace
 
+// Rows that a block of dnnopt_absmax_part takes at a time: four 16-byte loads
+// per thread are in flight, of one row, of two (up to 2048 columns) or of four
+// (up to 1024).
+__host__ __device__ __forceinline__ int absmax_rows(int cols) { return cols <= 1024 ? 4 : cols <= 2048 ? 2 : 1; }
+
 // Blocks [0, ga) take rows of A (M x K, stride lda), blocks [ga, grid) rows of
 // B (K x N, stride ldb); each stores the max |x| bits of its rows to part.
 // VEC: rows start on 16-byte boundaries (16-byte loads, four in flight per
 // thread).
+// What bounds it: HBM for large operands; for small ones the number of loads
+// that follow one another in a block.  With one row at a time and a block per
+// 64 KB, 9 x 768 x 768 was a chain of 20 rows per block on 38 blocks; with
+// rows taken together and a block per 8 KB it is one step (MI355X, us, the
+// launch: 768 x 768 10.8 -> 3.2, 130 x 4096 with A off 16-byte rows 25.1 ->
+// 4.8, 4096 x 4096 12.0 either way, 5.6 TB/s).
 template <int VEC>
 __global__ __launch_bounds__(256) void dnnopt_absmax_part(const float* __restrict__ A, int M, int K, int lda,
                                                          int ga, const float* __restrict__ B, int N, int ldb,
@@ -80,15 +91,17 @@ __global__ __launch_bounds__(256) void dnnopt_absmax_part(const float* __restric
     const int rows = is_a ? M : K, cols = is_a ? K : N, ld = is_a ? lda : ldb;
     const int g = is_a ? (int)blockIdx.x : (int)blockIdx.x - ga;
     const int G = is_a ? ga : (int)gridDim.x - ga;
+    const int R = absmax_rows(cols), sh = R == 4 ? 0 : R == 2 ? 1 : 2;  // load u: row u >> sh of the step
     unsigned m = 0;
-    for (int r = g; r < rows; r += G) {
-        const float* row = x + (size_t)r * ld;
+    for (long long r = (long long)g * R; r < rows; r += (long long)G * R) {
         for (int c0 = 0; c0 < cols; c0 += 256 * 16) {
             f32x4 v[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const int c = c0 + (u * 256 + (int)threadIdx.x) * 4;
-                v[u] = c < cols ? load4<VEC>(row, c, cols) : f32x4{0.f, 0.f, 0.f, 0.f};
+                const long long row = r + (u >> sh);
+                const int c = c0 + ((u & ((1 << sh) - 1)) * 256 + (int)threadIdx.x) * 4;
+                v[u] = row < rows && c < cols ? load4<VEC>(x + (size_t)row * ld, c, cols)
+                                              : f32x4{0.f, 0.f, 0.f, 0.f};
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u)
@@ -173,18 +186,21 @@ __global__ __launch_bounds__(256) void dnnopt_quantize_pair(const float* __restr
     }
 }
 
-// Blocks for the maxima of the two operands: about one per 64 KiB of input,
-// at most 1024 in all, shared out by size.
+// Blocks for the maxima of the two operands: about one per 8 KiB of input, at
+// most 1024 in all (one wave reduces them), shared out by size, none without
+// rows of its own.
 void absmax_blocks(int M, int N, int K, int* ga, int* gb) {
     const double a = (double)M * K, b = (double)K * N;
-    long long total = (long long)((a + b) * 4 / 65536) + 2;
+    long long total = (long long)((a + b) * 4 / 8192) + 2;
     if (total > 1024) total = 1024;
+    const int ra = absmax_rows(K), rb = absmax_rows(N);
+    const long long steps_a = ((long long)M + ra - 1) / ra, steps_b = ((long long)K + rb - 1) / rb;
     long long x = (long long)(total * a / (a + b));
     if (x < 1) x = 1;
-    if (x > M) x = M;
+    if (x > steps_a) x = steps_a;
     long long y = total - x;
     if (y < 1) y = 1;
-    if (y > K) y = K;
+    if (y > steps_b) y = steps_b;
     *ga = (int)x;
     *gb = (int)y;
 }
