@@ -296,6 +296,11 @@ int dnnopt_hip_plan_gemm_s8(int with_scale, int M, int N, int K, dnnopt_plan* ou
     return st;
 }
 
+// Wave groups that share the k of a 64 x 32 tile (launch_s8_q8b).
+static int q8b_groups(int M, int N) {
+    return (long long)((N + 31) / 32) * ((M + 63) / 64) <= num_cus() ? 2 : 1;
+}
+
 int dnnopt_hip_plan_gemm_int8_f32(int M, int N, int K, dnnopt_plan* out) {
     if (!out || !dims_ok(M, N, K)) return DNNOPT_ERR_INVALID_ARG;
     Launch L;
@@ -321,7 +326,7 @@ int dnnopt_hip_plan_gemm_int8_f32(int M, int N, int K, dnnopt_plan* out) {
         out->splits = 1;
         out->grid_x = xcd_grid((N + 31) / 32, (M + 63) / 64);
         out->grid_y = out->grid_z = 1;
-        out->block = 256;
+        out->block = 256 * q8b_groups(M, N);
         snprintf(out->name, sizeof out->name, "%s", "dnnopt_s8_lds_q8b");
         return DNNOPT_OK;
     }
@@ -638,7 +643,7 @@ int dnnopt_hip_gemm_int8_f32(int M, int N, int K, float alpha, const float* A, i
         a.qpart = part;
         a.ga = ga;
         a.gb = gb;
-        return finish_launch(launch_s8_q8b(dim3((unsigned)xcd_grid(a.tiles_n, a.tiles_m)), a, s));
+        return finish_launch(launch_s8_q8b(q8b_groups(M, N), dim3((unsigned)xcd_grid(a.tiles_n, a.tiles_m)), a, s));
     }
     if (N > 0x7FFFFFFF / 2 || (long long)N * ((K + 15) & ~15) > 0x7FFFFFFFll) return DNNOPT_ERR_UNSUPPORTED;
     // Staging (slot 1): [qA M x ldq][qB N x ldq][absmax partials][max|A|, max|B|];

@@ -265,10 +265,12 @@ __device__ __forceinline__ int swz16(int row, int c) { return c ^ (row & 7); }
 // of that column's LDS row: the LDS layout and the MFMAs are those of int8
 // B.  Columns past N hold whatever the loads return; their outputs are not
 // stored.
-template <int MT, int NT, int WM, int WN, int D, int EPI, int BK = 128, int QB = 0>
-__global__ __launch_bounds__(WM* WN * 64) void dnnopt_s8_lds(S8Args p) {
+// KG = 2: two groups of WM * WN waves, each with its own stages, take a half of
+// the k blocks each; their int32 sums are added in LDS.
+template <int MT, int NT, int WM, int WN, int D, int EPI, int BK = 128, int QB = 0, int KG = 1>
+__global__ __launch_bounds__(WM* WN * KG * 64) void dnnopt_s8_lds(S8Args p) {
     constexpr int BM = WM * MT * 16, BN = WN * NT * 16;  // BK: bytes (= k) per block
-    constexpr int NTH = WM * WN * 64;
+    constexpr int NTH = WM * WN * 64;  // threads of a k group
     constexpr int ROWB = BK;
     constexpr int CPR = ROWB / 16;  // 16-byte chunks per LDS row
     constexpr int KK = BK / 64;     // MFMA k-steps per block
@@ -276,21 +278,26 @@ __global__ __launch_bounds__(WM* WN * 64) void dnnopt_s8_lds(S8Args p) {
     constexpr int ACH = BM * CPR, BCH = BN * CPR;  // 16-byte chunks per block
     constexpr int AU = (ACH + NTH - 1) / NTH, BU = (BCH + NTH - 1) / NTH;
     constexpr int CROW = BN + 4;
-    constexpr int LDS_BYTES = 2 * STAGE > BM * CROW * 4 ? 2 * STAGE : BM * CROW * 4;
+    constexpr int LDS_BYTES = KG * 2 * STAGE > BM * CROW * 4 ? KG * 2 * STAGE : BM * CROW * 4;
     __shared__ __attribute__((aligned(16))) char lds[LDS_BYTES];
 
     const int lane = lane_id(), r = lane & 15, g = lane >> 4;
-    const int w = wave_id();
+    const int kg = KG > 1 ? wave_id() / (WM * WN) : 0;
+    const int w = wave_id() - kg * (WM * WN);
     const int wn = w % WN, wm = w / WN;
-    const int t = (int)threadIdx.x;
+    const int t = (int)threadIdx.x - kg * NTH;
     const TileXY tile = xcd_tile((int)blockIdx.x, p.tiles_n, p.tiles_m);
     if (!tile.ok) return;
     const int tile_n = tile.n, tile_m = tile.m, split = blockIdx.z;
     const int m0 = tile_m * BM, n0 = tile_n * BN;
 
     const int nblk = (p.K + BK - 1) / BK;
-    const int b_lo = (int)(((long long)nblk * split) / p.splits);
-    const int b_hi = (int)(((long long)nblk * (split + 1)) / p.splits);
+    const int s_lo = (int)(((long long)nblk * split) / p.splits);
+    const int s_hi = (int)(((long long)nblk * (split + 1)) / p.splits);
+    // KG = 2: group 0 takes the first half of the blocks (the larger one, so
+    // that its count, nbm, is every group's number of barriers).
+    const int nbm = (s_hi - s_lo + KG - 1) / KG;
+    const int b_lo = s_lo + kg * nbm, b_hi = KG > 1 && kg == 0 ? s_lo + nbm : s_hi;
 
     // Ranges end at the last byte of each operand, rounded up to a dword.
     const __amdgpu_buffer_rsrc_t ra =
@@ -352,7 +359,7 @@ __global__ __launch_bounds__(WM* WN * 64) void dnnopt_s8_lds(S8Args p) {
         }
     };
     auto write_stage = [&](int slot, int buf, int blk) {
-        char* St = lds + buf * STAGE;
+        char* St = lds + (2 * kg + buf) * STAGE;
         // Bytes of A past K (the next row's data) are zeroed in the block
         // that holds k = K - 1, which zeroes their products whatever B holds.
         const bool tail = (blk + 1) * BK > p.K;
@@ -398,7 +405,7 @@ __global__ __launch_bounds__(WM* WN * 64) void dnnopt_s8_lds(S8Args p) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = i32x4{0, 0, 0, 0};
     auto compute = [&](int buf) {
-        const char* St = lds + buf * STAGE;
+        const char* St = lds + (2 * kg + buf) * STAGE;
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
             i32x4 af[MT], bfr[NT];
@@ -415,19 +422,19 @@ __global__ __launch_bounds__(WM* WN * 64) void dnnopt_s8_lds(S8Args p) {
     };
 
     const int nb = b_hi - b_lo;
-    if (nb > 0) {
+    if (nbm > 0) {
 #pragma unroll
         for (int d = 0; d < D; ++d) load_stage(b_lo + d, d);
         write_stage(0, 0, b_lo);
     }
     __syncthreads();
     int i0 = 0;
-    for (; i0 + D <= nb; i0 += D) {
+    for (; i0 + D <= nbm; i0 += D) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             const int i = i0 + d;
             load_stage(b_lo + i + D, d);
-            compute(i & 1);
+            if (KG == 1 || i < nb) compute(i & 1);
             write_stage((d + 1) % D, (i + 1) & 1, b_lo + i + 1);
             __syncthreads();
         }
@@ -435,23 +442,31 @@ __global__ __launch_bounds__(WM* WN * 64) void dnnopt_s8_lds(S8Args p) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
         const int i = i0 + d;
-        if (i < nb) {
-            compute(i & 1);
+        if (i < nbm) {
+            if (KG == 1 || i < nb) compute(i & 1);
             write_stage((d + 1) % D, (i + 1) & 1, b_lo + i + 1);
             __syncthreads();
         }
     }
 
-    // Stage the accumulators in LDS (row-major tile), then write whole rows.
+    // Stage the accumulators in LDS (row-major tile; the second group adds its
+    // sums to the first's), then write whole rows.
     int32_t* Cs = reinterpret_cast<int32_t*>(lds);
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int h = 0; h < KG; ++h) {
+        if (kg == h) {
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
+            for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                Cs[((wm * MT + mt) * 16 + 4 * g + i) * CROW + (wn * NT + nt) * 16 + r] = acc[mt][nt][i];
-    __syncthreads();
+                for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        int32_t& c = Cs[((wm * MT + mt) * 16 + 4 * g + i) * CROW + (wn * NT + nt) * 16 + r];
+                        c = h ? c + acc[mt][nt][i] : acc[mt][nt][i];
+                    }
+        }
+        __syncthreads();
+    }
     constexpr int Q4 = BN / 4;
     if (p.splits > 1) {
         // Exact int32 partial tile [split][tile][BM * BN], summed by the
@@ -459,7 +474,7 @@ __global__ __launch_bounds__(WM* WN * 64) void dnnopt_s8_lds(S8Args p) {
         const int tiles = p.tiles_n * p.tiles_m;
         const int tile_id = tile_m * p.tiles_n + tile_n;
         int32_t* part = p.part + ((size_t)split * tiles + tile_id) * (BM * BN);
-        for (int e = t; e < BM * Q4; e += NTH) {
+        for (int e = (int)threadIdx.x; e < BM * Q4; e += KG * NTH) {
             const int row = e / Q4, q = e % Q4;
             *reinterpret_cast<i32x4*>(part + row * BN + 4 * q) = *reinterpret_cast<const i32x4*>(&Cs[row * CROW + 4 * q]);
         }
@@ -470,7 +485,7 @@ __global__ __launch_bounds__(WM* WN * 64) void dnnopt_s8_lds(S8Args p) {
     const __amdgpu_buffer_rsrc_t rc =
         make_rsrc(static_cast<char*>(p.C) + ((size_t)m0 * p.ldc + n0) * esz,
                   range31(((size_t)(p.M - 1 - m0) * p.ldc + (p.N - n0)) * esz));
-    for (int e = t; e < BM * Q4; e += NTH) {
+    for (int e = (int)threadIdx.x; e < BM * Q4; e += KG * NTH) {
         const int row = e / Q4, q = e % Q4;
         const int m = m0 + row, n = n0 + 4 * q;
         if (m >= p.M || n >= p.N) continue;
@@ -774,10 +789,19 @@ static hipError_t launch_s8_cfg(int cfg, dim3 grid, const S8Args& a, hipStream_t
     return hipGetLastError();
 }
 
-// 64 x 32 tiles, 3 blocks of 128 k in flight (MI355X, 128 x 4096 x 4096
-// call: 2 / 3 / 4 / 6 blocks 38.6 / 38.4 / 38.8 / 39.6 us).
-hipError_t launch_s8_q8b(dim3 grid, const S8Args& a, hipStream_t s) {
-    hipLaunchKernelGGL((dnnopt_s8_lds<2, 1, 2, 2, 3, 1, 128, 1>), grid, dim3(256), 0, s, a);
+// 64 x 32 tiles.  Up to one tile per CU (groups = 2): two groups of four waves share k, 2
+// blocks of 128 k in flight each, so that one group's quantization runs while
+// the other's loads arrive.  More tiles than that: one group, 3 blocks in
+// flight; the second tile of a CU fills the waits, and the larger workgroups
+// cost more than they give.  MI355X, us per call, one group -> two: 128 x 4096
+// x 4096 38.1 -> 35.9 (2 / 3 / 4 / 6 blocks with one group 38.6 / 38.4 / 38.8 /
+// 39.6), 16 x 4096 x 4096 36.1 -> 34.2, 256 x 2048 x 2048 24.5 -> 23.2, 512 x
+// 768 x 3072 35.8 -> 34.0; 470 tiles of 300 x 3000 x 1000 28.0 vs 29.0.
+hipError_t launch_s8_q8b(int groups, dim3 grid, const S8Args& a, hipStream_t s) {
+    if (groups == 2)
+        hipLaunchKernelGGL((dnnopt_s8_lds<2, 1, 2, 2, 2, 1, 128, 1, 2>), grid, dim3(512), 0, s, a);
+    else
+        hipLaunchKernelGGL((dnnopt_s8_lds<2, 1, 2, 2, 3, 1, 128, 1>), grid, dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

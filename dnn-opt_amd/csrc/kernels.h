@@ -373,7 +373,7 @@ hipError_t launch_quant_a(const float* A, int lda, int M, int K, int ldq, const 
 // fp32-API int8 GEMM, M > 8: int8 A (qA) x fp32 K x N B quantized while it is
 // staged (64 x 32 tiles through LDS), dequantizing epilogue.  grid.x =
 // xcd_grid(ceil(N / 32), ceil(M / 64)).
-hipError_t launch_s8_q8b(dim3 grid, const S8Args& a, hipStream_t s);
+hipError_t launch_s8_q8b(int groups, dim3 grid, const S8Args& a, hipStream_t s);
 // Reduce skinny partials [split][M][ncols_pad] into C (epilogue applied);
 // tile t (of T, tile width tw) has splits_of_tile(t, G, T) partials.
 hipError_t launch_skinny_reduce(const float* part, int G, int T, int tw, int M, int N, int ncols_pad,
