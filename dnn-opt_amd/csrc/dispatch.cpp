@@ -38,6 +38,10 @@
 //     is 5% ahead of it, another tile or split, up to k_pp.hip's 256 x 256.
 //   * bf16 storage with more than 64 rows and K a multiple of 8: k_pp.hip's
 //     tiles where their cost model is 5% ahead of the other tiles.
+//   * fp32, A stored M x K, more than 32 rows (K x N B: more than 128):
+//     k_wavek.hip's tiles where their cost model is 10% ahead.
+//   * bf16 from fp32 inputs: A, or A and B, rounded ahead into workspace where
+//     the models of the tiles that read them are ahead (plan_bf16_copies).
 //   The LDS-staged tile and k-split of bf16 storage above M = 128, and of
 //   fp32 inputs above M = 64, come from a fitted cost model (pick_tile) when
 //   it beats the rule by 5%; the fp32 register tile and k-split (A stored
