@@ -918,6 +918,14 @@ static int plan_s8_kernels(int epi, int M, int N, int K, Launch* L, bool lds_ok,
     long long model_splits = 0;
     const int forced_splits = tunable(kTuneS8Splits);
     const bool pp_ok = K % 16 == 0 && 256LL * ldc * 4 < 0x7FFFFFFFll;
+    // The tiles address A and B from their first row with 32-bit offsets: a
+    // long row stride leaves the lower tiles only (4096 x 4096 x 8 400 000
+    // takes 64 x 64, whose limit is a stride of 33 M; 256 x 256 stops at 8.4 M).
+    const auto spans_ok = [&](int k) {
+        const S8Config t = s8_config(k);
+        return (long long)t.wm * t.mt * 16 * (lda > 0 ? lda : K) + K < 0x7FFFFFFFll &&
+               (long long)t.wn * t.nt * 16 * (ldb > 0 ? ldb : K) + K < 0x7FFFFFFFll;
+    };
     if (M > 16) {
         const long long cus_ = num_cus();
         if (ceil_div(M, 64) * ceil_div(N, 64) >= cus_) cfg = 29;
@@ -929,21 +937,21 @@ static int plan_s8_kernels(int epi, int M, int N, int K, Launch* L, bool lds_ok,
             *bm_ = t.wm * t.mt * 16;
             *bn_ = t.wn * t.nt * 16;
             *kb_ = t.kblk;
-            return true;
+            return spans_ok(k);
         };
-        int bm0 = 0, bn0 = 0, kb0 = 0;
-        shape(cfg, &bm0, &bn0, &kb0);
+        const S8Config d = s8_config(cfg);
         const WgFit* def = nullptr;
         for (const WgFit& f : kS8Fit)
             if (f.cfg == cfg) def = &f;
-        const double def_us = wg_cost(kS8Model, *def, bm0, bn0, kb0, s8_rule_splits(cfg, M, N, K), M, N, K, cus_);
+        const double def_us = wg_cost(kS8Model, *def, d.wm * d.mt * 16, d.wn * d.nt * 16, d.kblk,
+                                      s8_rule_splits(cfg, M, N, K), M, N, K, cus_);
         const TilePick pick = best_wg_tile(kS8Model, M, N, K, shape);
-        if (forced_cfg < 0 && pick.us < 0.95 * def_us) {
+        if (forced_cfg < 0 && pick.s > 0 && pick.us < 0.95 * def_us) {
             cfg = pick.cfg;
             model_splits = pick.s;
         }
     }
-    if (forced_cfg >= 0 && forced_cfg < s8_config_count() && (forced_cfg < kS8PPFirst || pp_ok)) cfg = forced_cfg;
+    if (forced_cfg >= 0 && forced_cfg < s8_config_count() && (forced_cfg < kS8PPFirst || (pp_ok && spans_ok(forced_cfg)))) cfg = forced_cfg;
     if (cfg >= kS8FirstLds && !lds_ok) cfg = M <= 16 ? 5 : (M >= 128 ? 3 : 2);
     const bool lds = cfg >= kS8FirstLds;
     const bool dma = cfg >= kS8FirstDma;
@@ -967,9 +975,7 @@ static int plan_s8_kernels(int epi, int M, int N, int K, Launch* L, bool lds_ok,
     }
     if (forced_splits > 0) s = std::min<long long>(forced_splits, std::max<long long>(1, nblk / c.kw));
     if (s > 1 && tiles > kMaxTickets && !split_reduce_mode() && !lds) s = 1;
-    // The tiles address A and B from their first row with 32-bit offsets.
-    if ((long long)bm * (lda > 0 ? lda : K) + K >= 0x7FFFFFFFll || (long long)bn * (ldb > 0 ? ldb : K) + K >= 0x7FFFFFFFll)
-        return DNNOPT_ERR_UNSUPPORTED;
+    if (!spans_ok(cfg)) return DNNOPT_ERR_UNSUPPORTED;
     if (tm > 65535 || s > 65535 || tn * tm > 0x7FFFFFF0ll) return DNNOPT_ERR_UNSUPPORTED;
     // The LDS-staged kernel always hands its k-splits to the reduce kernel.
     L->defer_reduce = (s > 1 && (split_reduce_mode() || lds)) ? 1 : 0;

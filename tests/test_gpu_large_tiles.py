@@ -105,6 +105,20 @@ def test_planned_by_size_and_k_alignment(lib):
             assert (p["rows"], p["cols"]) not in large, p
 
 
+@pytest.mark.parametrize("M,N,K", [(4096, 4096, 8400000), (2048, 1024, 8400000), (1024, 1024, 17000000),
+                                   (256, 64, 8388608), (2048, 4096, 16777200), (128, 128, 16777216)])
+def test_int8_long_rows_keep_tiles(lib, M, N, K):
+    """Tiles of 128 and 256 rows cannot reach rows of 8.4 M or 16.8 M bytes with
+    32-bit offsets; the lower int8 tiles can, and such a call stays on tiles,
+    also when a large tile is forced."""
+    b = u.binding()
+    for cfg in (-1, S8_FIRST):
+        with lib.tunables(S8_CFG=cfg):
+            p = lib.plan_s8(M, N, K)
+            assert p["kernel"] == b.K_MFMA_S8, p
+            assert p["rows"] * K + K < 2**31 - 1 and p["cols"] * K + K < 2**31 - 1, p
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["bf16", "s8"])
 def test_wide_c_stride_keeps_other_tiles(lib, orc, dev, kind):
