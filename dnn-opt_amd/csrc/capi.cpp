@@ -271,6 +271,19 @@ int dnnopt_hip_plan_gemm_bf16(int fp32_inputs, int M, int N, int K, dnnopt_plan*
     return st;
 }
 
+int dnnopt_hip_plan_gemm_bf16_copies(int M, int N, int K, dnnopt_plan* out, int* operands) {
+    if (!out || !operands || !dims_ok(M, N, K)) return DNNOPT_ERR_INVALID_ARG;
+    Launch L;
+    int st = plan_bf16(1, M, N, K, K, N, &L);
+    if (st != DNNOPT_OK) return st;
+    Bf16Copies cp{};
+    const bool copies = plan_bf16_copies(L, M, N, K, K, N, N, &cp);
+    *operands = copies ? (cp.both ? 2 : 1) : 0;
+    *out = copies ? cp.L.pub : L.pub;
+    if (copies) out->workspace_bytes = cp.bytes + cp.L.part_bytes;
+    return DNNOPT_OK;
+}
+
 int dnnopt_hip_plan_gemm_bf16_ex(int transA, int transB, int M, int N, int K, dnnopt_plan* out) {
     if (!out || !dims_ok(M, N, K) || (transA != 0 && transA != 1) || (transB != 0 && transB != 1))
         return DNNOPT_ERR_INVALID_ARG;

@@ -698,6 +698,10 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
             }
         }
         const bool forced_dma = forced_cfg >= kTileFirstDma && forced_cfg < kTileF32Few;
+        // A forced launch on copies (make_bf16_copies): the tiles that round
+        // while staging, in the same blocks of k.
+        if (mode == kTileF2B && tile_a16(forced_cfg)) cfg = forced_cfg == kTileA16Tall && tall_ok ? kTileF2BTall : 20;
+        if (mode == kTileF2B && tile_pp(forced_cfg) && tall_ok) cfg = kTileF2BTall;
         if (((forced_cfg >= kTileFirstLds && forced_cfg < kTileF32Few) || forced_cfg == kTileBF16Tb48 ||
              forced_cfg == kTileBF16Tb48Few || forced_cfg == kTileBF16Dma4w ||
              (tile_pp(forced_cfg) && mode == kTileBF16 && K % 8 == 0 && tall_ok) || (forced_cfg == kTileF2BTall && tall_ok)) &&
@@ -1253,8 +1257,27 @@ int plan_s8(int epi, int M, int N, int K, Launch* L, bool lds_ok, int lda, int l
 // Tiles of a bf16 A and an fp32 B (kTileA16): 128 x 96 with 128 k per block,
 // 256 x 96 with 64, 1 or 2 k-splits (40 shapes, M = 34..2048, N = 768..11008,
 // K = 768..4096, 143 points: median error 5%, 90% within 12%).
-static const WgFit kA16Fit[] = {{20, 1, 3.505, 1.426, 0.0}, {kTileF2BTall, 1, 3.243, 1.049, 0.0}};
+static const WgFit kA16Fit[] = {{kTileA16Wide, 1, 3.505, 1.426, 0.0}, {kTileA16Tall, 1, 3.243, 1.049, 0.0}};
 static const WgModel kA16Model{kA16Fit, 2, 0, 3.812, 2.503, 0.152, 0.0};
+
+// The launch of LDS-staged configuration `cfg` with `s` k-splits, summed by the
+// reduce kernel.
+static Launch staged_launch(int mode, int cfg, long long s, int M, int N) {
+    const TileConfig c = tile_config(cfg);
+    Launch L;
+    L.mode = mode;
+    L.cfg = cfg;
+    L.bm = c.wm * c.mt * 16;
+    L.bn = c.wn * c.nt * 16;
+    L.tn = (int)ceil_div(N, L.bn);
+    L.tm = (int)ceil_div(M, L.bm);
+    L.grid = dim3((unsigned)xcd_grid(L.tn, L.tm), 1, (unsigned)s);
+    L.defer_reduce = s > 1 ? 1 : 0;
+    L.part_bytes = s > 1 ? (size_t)s * L.tn * L.tm * L.bm * L.bn * sizeof(float) : 0;
+    fill_pub(&L, DNNOPT_K_TILE_BF16, tile_pp(cfg) ? "dnnopt_tile_bf16_dma" : "dnnopt_tile_bf16_lds", L.bm, L.bn, (int)s,
+             c.wm * c.wn * c.kw * 64);
+    return L;
+}
 
 // Rounding operands once, into workspace, ahead of the tiles (6 bytes of
 // traffic per element at 6.3 TB/s) against tiles that round every element each
@@ -1266,20 +1289,26 @@ static const WgModel kA16Model{kA16Fit, 2, 0, 3.812, 2.503, 0.152, 0.0};
 // 1632 x 4352 x 3520 142.5 / 120.5 / 83.4, 300 x 1001 x 1003 10.5 / 17.7 / -.
 // The direct tiles run at 0.9 of their model's times (0.77..1.16 on those
 // shapes; the fit predates their raw register ring); the other two have to be
-// 5% and 10% ahead.
+// 5% and 10% ahead.  Tunable TILE_CFG forces either (kTileA16Wide, kTileA16Tall
+// or one of k_pp.hip's tiles, with the direct plan's splits).
 static bool make_bf16_copies(const Launch& direct, int M, int N, int K, int lda, int ldb, int ldc, Bf16Copies* out) {
     if (ldc <= 0) ldc = N;
-    if (direct.est_us <= 0.0 || M <= 64 || (long long)lda * 16 >= 0x7FFFFFFFll || (long long)ldb * 16 >= 0x7FFFFFFFll)
+    const int forced_cfg = tunable(kTuneTileCfg);
+    const bool force_a = tile_a16(forced_cfg), force_both = tile_pp(forced_cfg), forced = force_a || force_both;
+    if (direct.mode != kTileF2B || direct.cfg < kTileFirstLds || direct.family != DNNOPT_K_TILE_BF16) return false;
+    if ((!forced && (direct.est_us <= 0.0 || M <= 64)) || (long long)lda * 16 >= 0x7FFFFFFFll ||
+        (long long)ldb * 16 >= 0x7FFFFFFFll)
         return false;
     const long long k8 = ((long long)K + 7) & ~7ll, n8 = ((long long)N + 7) & ~7ll;
-    const size_t a = ((size_t)M * k8 * 2 + 255) & ~(size_t)255, b = (size_t)k8 * n8 * 2;
+    const size_t a = ((size_t)M * k8 * 2 + 255) & ~(size_t)255, b = ((size_t)k8 * n8 * 2 + 255) & ~(size_t)255;
     if (k8 > 0x7FFFFFF0ll || n8 > 0x7FFFFFF0ll) return false;
+    // The direct plan's spans (B, and A in fp32) fit 32-bit offsets; so must
+    // 256 rows of C.
+    const bool tall_ok = 256LL * ldc * 4 < 0x7FFFFFFFll;
     out->lda = (int)k8;
     double best = 0.90 * direct.est_us;
     bool found = false;
-    // The direct plan's spans (B, and A in fp32) fit 32-bit offsets; so must
-    // 256 rows of C.
-    if (a <= kOptionalBytes && 256LL * ldc * 4 < 0x7FFFFFFFll) {
+    if (a <= kOptionalBytes && tall_ok && !force_both) {
         const TilePick t = best_wg_tile(kA16Model, M, N, K, [&](int k, int* bm_, int* bn_, int* kb_) {
             const TileConfig c = tile_config(k);
             *bm_ = c.wm * c.mt * 16;
@@ -1288,19 +1317,8 @@ static bool make_bf16_copies(const Launch& direct, int M, int N, int K, int lda,
             return true;
         });
         const double us = t.us + (double)M * K * 6e-6 / 6.3;
-        if (t.s > 0 && us < 0.95 * best) {
-            const TileConfig c = tile_config(t.cfg);
-            Launch& L = out->L;
-            L = Launch{};
-            L.mode = kTileA16;
-            L.cfg = t.cfg;
-            L.bm = c.wm * c.mt * 16;
-            L.bn = c.wn * c.nt * 16;
-            L.tn = (int)ceil_div(N, L.bn);
-            L.tm = (int)ceil_div(M, L.bm);
-            L.grid = dim3((unsigned)xcd_grid(L.tn, L.tm), 1, (unsigned)t.s);
-            L.defer_reduce = t.s > 1 ? 1 : 0;
-            L.part_bytes = t.s > 1 ? (size_t)t.s * L.tn * L.tm * L.bm * L.bn * sizeof(float) : 0;
+        if (force_a || (t.s > 0 && us < 0.95 * best)) {
+            out->L = force_a ? staged_launch(kTileA16, forced_cfg, direct.grid.z, M, N) : staged_launch(kTileA16, t.cfg, t.s, M, N);
             out->both = false;
             out->K = K;
             out->a_bytes = out->bytes = a;
@@ -1308,11 +1326,16 @@ static bool make_bf16_copies(const Launch& direct, int M, int N, int K, int lda,
             found = true;
         }
     }
+    if (force_a) return found;
     const double copy_us = 5.0 + ((double)M * K + (double)K * N) * 6e-6 / 6.3;
     Launch two;
-    if (a + b <= kOptionalBytes && copy_us < best &&
-        plan_bf16(0, M, N, (int)k8, (int)k8, (int)n8, &two, 0, ldc) == DNNOPT_OK && two.est_us > 0.0 &&
-        copy_us + two.est_us < 0.9 * best) {
+    if (force_both) {
+        if (tall_ok) two = staged_launch(kTileBF16, forced_cfg, direct.grid.z, M, N);
+    } else if (copy_us >= best || plan_bf16(0, M, N, (int)k8, (int)k8, (int)n8, &two, 0, ldc) != DNNOPT_OK ||
+               two.est_us <= 0.0 || copy_us + two.est_us >= 0.9 * best) {
+        return found;
+    }
+    if (a + b <= kOptionalBytes && two.family == DNNOPT_K_TILE_BF16) {
         out->L = two;
         out->both = true;
         out->K = (int)k8;

@@ -1367,6 +1367,9 @@ static const TileConfig kTileConfigs[] = {
     {4, 2, 1, 1, 4, 3, 64},   // 62: 64 x 32
     {2, 3, 1, 1, 4, 3, 64},   // 63: 32 x 48
     {2, 4, 1, 1, 4, 3, 64},   // 64: 32 x 64
+    // bf16 A, fp32 B (kTileA16): {MT, NT, WM, WN, 1, depth, k per block}
+    {2, 3, 4, 2, 1, 2, 128},  // 65: 128 x 96
+    {4, 3, 4, 2, 1, 2, 64},   // 66: 256 x 96
 };
 
 int tile_config_count() { return (int)(sizeof(kTileConfigs) / sizeof(kTileConfigs[0])); }
@@ -1421,8 +1424,8 @@ TileConfig tile_config(int idx) { return kTileConfigs[idx]; }
 // A bf16, B fp32 (kTileA16).  A third block in the register ring measured 1%
 // slower on both (256 x 96: 87.4 vs 88.1 us at 512 x 11008 x 4096).
 static hipError_t launch_tile_a16(int cfg_idx, dim3 grid, const TileArgs& a, hipStream_t s) {
-    if (cfg_idx == 20) hipLaunchKernelGGL((dnnopt_tile_bf16_lds<2, 3, 4, 2, 2, kTileA16, 0, 128, 1, 1>), grid, dim3(512), 0, s, a);
-    else if (cfg_idx == kTileF2BTall) hipLaunchKernelGGL((dnnopt_tile_bf16_lds<4, 3, 4, 2, 2, kTileA16, 0, 64, 1, 1>), grid, dim3(512), 0, s, a);
+    if (cfg_idx == kTileA16Wide) hipLaunchKernelGGL((dnnopt_tile_bf16_lds<2, 3, 4, 2, 2, kTileA16, 0, 128, 1, 1>), grid, dim3(512), 0, s, a);
+    else if (cfg_idx == kTileA16Tall) hipLaunchKernelGGL((dnnopt_tile_bf16_lds<4, 3, 4, 2, 2, kTileA16, 0, 64, 1, 1>), grid, dim3(512), 0, s, a);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
@@ -1434,7 +1437,8 @@ hipError_t launch_tile(int mode, int cfg_idx, int ta, int tb, int al, dim3 grid,
     if (cfg_idx < 0 || cfg_idx >= tile_config_count()) return hipErrorInvalidValue;
     if (tile_wavek(cfg_idx))
         return mode == kTileF32 && !ta ? launch_tile_f32_wavek(cfg_idx - kTileWavekFirst, tb, grid, a, s) : hipErrorInvalidValue;
-    if (mode == kTileA16) return launch_tile_a16(cfg_idx, grid, a, s);
+    if (mode == kTileA16 || tile_a16(cfg_idx))
+        return mode == kTileA16 ? launch_tile_a16(cfg_idx, grid, a, s) : hipErrorInvalidValue;
     if (tile_pp(cfg_idx)) {
         if (mode != kTileBF16 || !al) return hipErrorInvalidValue;
         PPArgs q{};

@@ -266,6 +266,11 @@ constexpr bool tile_pp(int cfg) { return cfg >= kTilePPFirst && cfg <= kTilePPLa
 // kTileWavekFirst + i is launch_tile_f32_wavek's i.
 constexpr int kTileWavekFirst = 58, kTileWavekLast = 64;
 constexpr bool tile_wavek(int cfg) { return cfg >= kTileWavekFirst && cfg <= kTileWavekLast; }
+// bf16 copy of A, fp32 B rounded while it is staged (mode kTileA16): 128 x 96
+// with 128 k per block and 256 x 96 with 64, the shapes and blocks of
+// configurations 20 and kTileF2BTall.
+constexpr int kTileA16Wide = 65, kTileA16Tall = 66;
+constexpr bool tile_a16(int cfg) { return cfg == kTileA16Wide || cfg == kTileA16Tall; }
 constexpr bool tile_f32_dma(int cfg) { return cfg >= kTileF32DmaFirst && cfg <= kTileF32DmaLast; }
 // k per LDS block of an LDS-staged configuration: its kblk (or
 // DNNOPT_LDS_KB) when both stages fit in 128 KiB of LDS, else 64.

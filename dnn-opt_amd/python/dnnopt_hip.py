@@ -94,6 +94,7 @@ C_ABI = {
     "dnnopt_hip_plan_sgemm": (_I, [_I, _I, _I, _I, _I, POINTER(Plan)]),
     "dnnopt_hip_plan_sgemm_ex": (_I, [_I, _I, _I, _I, _I, _I, _I, _I, POINTER(Plan)]),
     "dnnopt_hip_plan_gemm_bf16": (_I, [_I, _I, _I, _I, POINTER(Plan)]),
+    "dnnopt_hip_plan_gemm_bf16_copies": (_I, [_I, _I, _I, POINTER(Plan), POINTER(ctypes.c_int)]),
     "dnnopt_hip_plan_gemm_bf16_ex": (_I, [_I, _I, _I, _I, _I, POINTER(Plan)]),
     "dnnopt_hip_plan_gemm_s8": (_I, [_I, _I, _I, _I, POINTER(Plan)]),
     "dnnopt_hip_plan_gemm_int8_f32": (_I, [_I, _I, _I, POINTER(Plan)]),
@@ -264,6 +265,12 @@ class Lib:
         p = Plan()
         self._check(self.so.dnnopt_hip_plan_gemm_bf16(fp32_inputs, M, N, K, ctypes.byref(p)), "plan_bf16")
         return p.as_dict()
+
+    def plan_bf16_copies(self, M, N, K) -> dict:
+        """The GEMM launch of gemm_bf16_f32in; `operands`: 1 on a rounded copy of A, 2 of A and B, 0 on neither."""
+        p, n = Plan(), ctypes.c_int(-1)
+        self._check(self.so.dnnopt_hip_plan_gemm_bf16_copies(M, N, K, ctypes.byref(p), ctypes.byref(n)), "plan_bf16_copies")
+        return dict(p.as_dict(), operands=n.value)
 
     def plan_bf16_ex(self, M, N, K, transA=0, transB=0) -> dict:
         p = Plan()

@@ -244,12 +244,19 @@ int dnnopt_hip_plan_sgemm(int transA, int transB, int M, int N, int K,
  * operand with 32-bit offsets are only chosen when its strides allow. */
 int dnnopt_hip_plan_sgemm_ex(int transA, int transB, int M, int N, int K,
                              int lda, int ldb, int ldc, dnnopt_plan* out);
-/* fp32_inputs = 1: the launch that rounds the operands while staging them.  A
- * call with many rows may instead round A, or both operands, once into library
- * workspace and run the tiles on the copies (never while its stream is being
- * captured). */
+/* fp32_inputs = 1: the launch that rounds the operands while staging them
+ * (dnnopt_hip_plan_gemm_bf16_copies: the launch on rounded copies that a call
+ * with many rows makes instead). */
 int dnnopt_hip_plan_gemm_bf16(int fp32_inputs, int M, int N, int K,
                               dnnopt_plan* out);
+/* dnnopt_hip_gemm_bf16_f32in with unpadded strides: *operands = 1 where the
+ * call first rounds A into library workspace, 2 where it rounds A and B, 0
+ * where it rounds while staging; out = the GEMM launch (workspace_bytes: the
+ * copies and the launch's partials).  A call whose stream is being captured, or
+ * that finds no memory for the copies, makes dnnopt_hip_plan_gemm_bf16's launch
+ * instead. */
+int dnnopt_hip_plan_gemm_bf16_copies(int M, int N, int K, dnnopt_plan* out,
+                                     int* operands);
 int dnnopt_hip_plan_gemm_bf16_ex(int transA, int transB, int M, int N, int K,
                                  dnnopt_plan* out);
 int dnnopt_hip_plan_gemm_s8(int with_scale, int M, int N, int K,
@@ -304,7 +311,8 @@ int dnnopt_hip_device_count(void);    /* 0 when no device is visible        */
 #define DNNOPT_TUNE_TILE_CFG        10  /* force a tile configuration (bf16 LDS-staged: 5-34, 37-40, 51-57;
                                            fp32 register tiles: 1-4, 35, 36; fp32 LDS-DMA tiles,
                                            A stored M x K: 41-47, and 48-50 with B stored N x K;
-                                           four waves splitting k: 58-64) */
+                                           four waves splitting k: 58-64; bf16 from fp32 inputs
+                                           on copies of both operands: 51-57, of A: 65, 66) */
 #define DNNOPT_TUNE_TILE_TICKET     11
 #define DNNOPT_TUNE_S8_CFG          12
 #define DNNOPT_TUNE_S8_ROWDOT       13

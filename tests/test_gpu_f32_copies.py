@@ -131,3 +131,38 @@ def test_captured_after_a_warm_call(lib, orc, dev):
         torch.cuda.synchronize()
         g.replay()
         u.assert_fp32_close(host(dC), want, scale, K, f"replay {rep}")
+
+
+# TILE_CFG of a launch on copies -> (operands copied, rows, columns, TILE_CFG of the direct tiles with its blocks of k)
+FORCED = {65: (1, 128, 96, 20), 66: (1, 256, 96, 40), 51: (2, 256, 256, 40), 52: (2, 256, 192, 40),
+          53: (2, 256, 128, 40), 54: (2, 128, 128, 40), 55: (2, 128, 256, 40), 56: (2, 128, 192, 40), 57: (2, 256, 64, 40)}
+
+
+@pytest.mark.parametrize("cfg", sorted(FORCED))
+@pytest.mark.parametrize("splits", [1, 2])
+def test_every_tile_on_copies(lib, orc, dev, cfg, splits):
+    """Each tile that reads copies, at its edges (a k tail, odd strides, one
+    block of k, odd and even block counts): within the fp32 bound, and the bits
+    of the tiles that round while staging, with the same k-splits."""
+    operands, rows, cols, direct = FORCED[cfg]
+    for M, N, K, pad, alpha, beta in [(9, 64, 5, 1, 1.0, 0.0), (129, 97, 64, 0, 0.5, 1.0), (255, 193, 200, 3, 1.0, 0.0),
+                                      (257, 300, 391, 2, -2.0, 0.25), (300, 515, 1001, 0, 1.0, 1.0)]:
+        A, B = u.normal(orc, M * K, 1).reshape(M, K), u.normal(orc, K * N, 2, 0, 0.02).reshape(K, N)
+        sa, sb = np.full((M, K + pad), np.nan, np.float32), np.full((K, N + pad), np.nan, np.float32)
+        sa[:, :K], sb[:, :N] = A, B
+        C0 = u.uniform(orc, M * N, 3).reshape(M, N)
+        want, scale = u.exact(u.bf16_value(u.bf16_bits(orc, A)), u.bf16_value(u.bf16_bits(orc, B)), alpha, beta, C0)
+        dA, dB = dev_copy(sa, dev), dev_copy(sb, dev)
+        got = []
+        for c in (cfg, direct):
+            dC = dev_copy(C0 if beta else np.full_like(C0, np.nan), dev)
+            with lib.tunables(TILE_CFG=c, TILE_SPLITS=splits):
+                p = lib.plan_bf16_copies(M, N, K)
+                if c == cfg:
+                    assert (p["operands"], p["rows"], p["cols"], p["block"]) == (operands, rows, cols, 512), p
+                else:
+                    assert p["operands"] == 0, p
+                lib.gemm_bf16_f32in(M, N, K, alpha, dA, K + pad, dB, N + pad, beta, dC, N, stream=stream())
+            got.append(host(dC))
+        u.assert_fp32_close(got[0], want, scale, K, f"{cfg} {M}x{N}x{K} splits={splits}")
+        u.assert_bits_equal(got[0], got[1], f"{cfg} and {direct} {M}x{N}x{K} splits={splits}")

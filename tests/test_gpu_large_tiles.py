@@ -85,6 +85,25 @@ def test_s8_tiles(lib, orc, dev, tile, scaled):
                 assert np.array_equal(host(dC), acc.astype(np.int32)), (TILES[tile], M, N, K)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", range(len(TILES)))
+def test_s8_tiles_dynamic_scale(lib, orc, dev, tile):
+    """The dequantizing epilogue of the fp32-input int8 GEMM on these tiles
+    (quantized copies of both operands): the oracle's bits."""
+    for M, N, K, _, splits, _, _ in SHAPES:
+        M, K = max(M, 9), 16 * ((K + 15) // 16) * (2 if K > 64 else 1)
+        A, B, C0 = u.uniform(orc, M * K, 1), u.uniform(orc, K * N, 2), u.uniform(orc, M * N, 3)
+        for beta in (0.0, 0.5):
+            want = C0.copy()
+            orc.orc_gemm_int8(M, N, K, 0.75, u.ptr(A), K, u.ptr(B), N, beta, u.ptr(want), N)
+            dC = dev_copy(C0 if beta else np.full_like(C0, np.nan), dev)
+            with lib.tunables(Q8B=0, S8_CFG=S8_FIRST + tile, S8_SPLITS=splits):
+                p = lib.plan_s8(M, N, K, with_scale=1)
+                assert (p["rows"], p["cols"], p["block"]) == (*TILES[tile], 512), p
+                lib.gemm_int8_f32(M, N, K, 0.75, dev_copy(A, dev), K, dev_copy(B, dev), N, beta, dC, N, stream=stream())
+            u.assert_bits_equal(host(dC), want, f"{TILES[tile]} {M}x{N}x{K} beta={beta}")
+
+
 def test_planned_by_size_and_k_alignment(lib):
     """Many-row shapes take the large tiles (bf16 2048 x 11008 x 4096 225 ->
     171 us, int8 1024 x 11008 x 4096 100 -> 49 us on MI355X); a K off whole
