@@ -495,10 +495,11 @@ static double wg_cost(const WgModel& md, const WgFit& f, int bm, int bn, int kb,
 }
 
 // The model's best configuration and split (1, 2 or 4, while the workgroups
-// stay within about one round: more splits than that only add partials).
+// stay within about one round: more splits than that only add partials), or
+// its best configuration with `fixed` splits.
 // shape(cfg, &bm, &bn, &kb) says whether a configuration may be used.
 template <class Shape>
-static TilePick best_wg_tile(const WgModel& md, int M, int N, int K, Shape shape) {
+static TilePick best_wg_tile(const WgModel& md, int M, int N, int K, Shape shape, long long fixed = 0) {
     const long long cus = num_cus();
     TilePick best{0, 0, 0.0};
     for (int i = 0; i < md.n; ++i) {
@@ -506,6 +507,11 @@ static TilePick best_wg_tile(const WgModel& md, int M, int N, int K, Shape shape
         int bm = 0, bn = 0, kb = 0;
         if (!shape(f.cfg, &bm, &bn, &kb)) continue;
         const long long tiles = ceil_div(M, bm) * ceil_div(N, bn), nblk = ceil_div(K, kb);
+        if (fixed > 0) {
+            const double us = wg_cost(md, f, bm, bn, kb, fixed, M, N, K, cus);
+            if (best.s == 0 || us < best.us) best = TilePick{f.cfg, fixed, us};
+            continue;
+        }
         for (long long s : {1, 2, 4}) {
             if (s > 1 && (s > nblk || s > max_splits() || tiles * s > cus + cus / 8)) break;
             const double us = wg_cost(md, f, bm, bn, kb, s, M, N, K, cus);
@@ -1279,6 +1285,26 @@ static Launch staged_launch(int mode, int cfg, long long s, int M, int N) {
     return L;
 }
 
+// k per block of an LDS-staged configuration.
+static long long staged_bk(int cfg) {
+    const TileConfig c = tile_config(cfg);
+    return tile_lds_bk(c.wm * c.mt * 16, c.wn * c.nt * 16, c.kblk);
+}
+
+// Whether two LDS-staged configurations with `s` k-splits each sum the same
+// ranges of k in the same order: every split starts at the same k, and no
+// workgroup divides its blocks between wave groups.  (Within a range each
+// output is one chain of 32-k MFMAs, k ascending, whatever the tile, and the
+// reduce kernel adds the splits in order, so the results then have the same
+// bits.)
+static bool same_sums(int cfg1, int cfg2, long long s, int K) {
+    if (tile_config(cfg1).kw != 1 || tile_config(cfg2).kw != 1) return false;
+    const long long kb1 = staged_bk(cfg1), kb2 = staged_bk(cfg2), n1 = ceil_div(K, kb1), n2 = ceil_div(K, kb2);
+    for (long long z = 1; z < s; ++z)
+        if (n1 * z / s * kb1 != n2 * z / s * kb2) return false;
+    return true;
+}
+
 // Rounding operands once, into workspace, ahead of the tiles (6 bytes of
 // traffic per element at 6.3 TB/s) against tiles that round every element each
 // time they stage it.  A alone costs one short launch and halves the bytes of
@@ -1291,6 +1317,9 @@ static Launch staged_launch(int mode, int cfg, long long s, int M, int N) {
 // shapes; the fit predates their raw register ring); the other two have to be
 // 5% and 10% ahead.  Tunable TILE_CFG forces either (kTileA16Wide, kTileA16Tall
 // or one of k_pp.hip's tiles, with the direct plan's splits).
+// A call under capture, or short of memory, takes the direct launch, so only
+// launches with the direct one's sums are candidates: the same call has the
+// same bits on either route.
 static bool make_bf16_copies(const Launch& direct, int M, int N, int K, int lda, int ldb, int ldc, Bf16Copies* out) {
     if (ldc <= 0) ldc = N;
     const int forced_cfg = tunable(kTuneTileCfg);
@@ -1299,26 +1328,31 @@ static bool make_bf16_copies(const Launch& direct, int M, int N, int K, int lda,
     if ((!forced && (direct.est_us <= 0.0 || M <= 64)) || (long long)lda * 16 >= 0x7FFFFFFFll ||
         (long long)ldb * 16 >= 0x7FFFFFFFll)
         return false;
-    const long long k8 = ((long long)K + 7) & ~7ll, n8 = ((long long)N + 7) & ~7ll;
+    const long long k8 = ((long long)K + 7) & ~7ll, n8 = ((long long)N + 7) & ~7ll, splits = direct.grid.z;
     const size_t a = ((size_t)M * k8 * 2 + 255) & ~(size_t)255, b = ((size_t)k8 * n8 * 2 + 255) & ~(size_t)255;
-    if (k8 > 0x7FFFFFF0ll || n8 > 0x7FFFFFF0ll) return false;
+    if (k8 > 0x7FFFFFF0ll || n8 > 0x7FFFFFF0ll || (splits > 1 && !direct.defer_reduce)) return false;
     // The direct plan's spans (B, and A in fp32) fit 32-bit offsets; so must
     // 256 rows of C.
-    const bool tall_ok = 256LL * ldc * 4 < 0x7FFFFFFFll;
+    if (256LL * ldc * 4 >= 0x7FFFFFFFll) return false;
+    const auto shape = [&](int k, int* bm_, int* bn_, int* kb_) {
+        const TileConfig c = tile_config(k);
+        *bm_ = c.wm * c.mt * 16;
+        *bn_ = c.wn * c.nt * 16;
+        *kb_ = (int)staged_bk(k);
+        return (!forced || k == forced_cfg) && same_sums(k, direct.cfg, splits, K);
+    };
     out->lda = (int)k8;
-    double best = 0.90 * direct.est_us;
+    double best = forced ? 1e30 : 0.90 * direct.est_us;
     bool found = false;
-    if (a <= kOptionalBytes && tall_ok && !force_both) {
-        const TilePick t = best_wg_tile(kA16Model, M, N, K, [&](int k, int* bm_, int* bn_, int* kb_) {
-            const TileConfig c = tile_config(k);
-            *bm_ = c.wm * c.mt * 16;
-            *bn_ = c.wn * c.nt * 16;
-            *kb_ = tile_lds_bk(*bm_, *bn_, c.kblk);
-            return true;
-        });
+    // A alone with more splits than the model was fitted on: from 129 rows
+    // (MI355X, us, direct -> A with 3 to 6 splits: 608 x 2677 x 3968 70.4 ->
+    // 61.1, 144 x 3885 x 3776 45.8 -> 41.6, 176 x 6464 x 3767 45.5 -> 45.3, but
+    // 96 x 4160 x 3392 22.1 vs 23.4 and 94 x 3789 x 3520 20.9 vs 21.8).
+    if (a <= kOptionalBytes && (forced || splits <= 2 || M > 128)) {
+        const TilePick t = best_wg_tile(kA16Model, M, N, K, shape, splits);
         const double us = t.us + (double)M * K * 6e-6 / 6.3;
-        if (force_a || (t.s > 0 && us < 0.95 * best)) {
-            out->L = force_a ? staged_launch(kTileA16, forced_cfg, direct.grid.z, M, N) : staged_launch(kTileA16, t.cfg, t.s, M, N);
+        if (t.s > 0 && us < 0.95 * best) {
+            out->L = staged_launch(kTileA16, t.cfg, splits, M, N);
             out->both = false;
             out->K = K;
             out->a_bytes = out->bytes = a;
@@ -1326,23 +1360,26 @@ static bool make_bf16_copies(const Launch& direct, int M, int N, int K, int lda,
             found = true;
         }
     }
-    if (force_a) return found;
     const double copy_us = 5.0 + ((double)M * K + (double)K * N) * 6e-6 / 6.3;
-    Launch two;
-    if (force_both) {
-        if (tall_ok) two = staged_launch(kTileBF16, forced_cfg, direct.grid.z, M, N);
-    } else if (copy_us >= best || plan_bf16(0, M, N, (int)k8, (int)k8, (int)n8, &two, 0, ldc) != DNNOPT_OK ||
-               two.est_us <= 0.0 || copy_us + two.est_us >= 0.9 * best) {
-        return found;
-    }
-    if (a + b <= kOptionalBytes && two.family == DNNOPT_K_TILE_BF16) {
-        out->L = two;
-        out->both = true;
-        out->K = (int)k8;
-        out->ldb = (int)n8;
-        out->a_bytes = a;
-        out->bytes = a + b;
-        found = true;
+    if (a + b <= kOptionalBytes && copy_us < best) {
+        // The bf16-storage plan of the copies where it has these sums, else
+        // k_pp.hip's best tile that has.
+        Launch two;
+        if (forced || plan_bf16(0, M, N, (int)k8, (int)k8, (int)n8, &two, 0, ldc) != DNNOPT_OK || two.est_us <= 0.0 ||
+            two.grid.z != splits || (splits > 1 && !two.defer_reduce) || !same_sums(two.cfg, direct.cfg, splits, K)) {
+            const TilePick t = best_wg_tile(kBf16PPModel, M, N, K, shape, splits);
+            two = t.s > 0 ? staged_launch(kTileBF16, t.cfg, splits, M, N) : Launch{};
+            two.est_us = t.us;
+        }
+        if (two.family == DNNOPT_K_TILE_BF16 && copy_us + two.est_us < 0.9 * best) {
+            out->L = two;
+            out->both = true;
+            out->K = (int)k8;
+            out->ldb = (int)n8;
+            out->a_bytes = a;
+            out->bytes = a + b;
+            found = true;
+        }
     }
     return found;
 }

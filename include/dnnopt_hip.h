@@ -254,7 +254,8 @@ int dnnopt_hip_plan_gemm_bf16(int fp32_inputs, int M, int N, int K,
  * where it rounds while staging; out = the GEMM launch (workspace_bytes: the
  * copies and the launch's partials).  A call whose stream is being captured, or
  * that finds no memory for the copies, makes dnnopt_hip_plan_gemm_bf16's launch
- * instead. */
+ * instead, with the same bits: a launch on copies sums k in the same ranges and
+ * order. */
 int dnnopt_hip_plan_gemm_bf16_copies(int M, int N, int K, dnnopt_plan* out,
                                      int* operands);
 int dnnopt_hip_plan_gemm_bf16_ex(int transA, int transB, int M, int N, int K,

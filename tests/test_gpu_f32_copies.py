@@ -25,8 +25,8 @@ def stream():
     return torch.cuda.current_stream().cuda_stream
 
 
-# The models round A alone (128 x 96 tiles, 256 x 96 tiles, a k-split) or both
-# operands (from about 700 rows) on these; the last two keep the direct tiles.
+# The models round A alone on some of these (tests/test_copies_routes.py says which),
+# the others keep the tiles that round while staging.
 SHAPES = [(200, 9000, 1000, 0, 1.0, 0.0), (380, 10007, 777, 3, 0.5, 1.0), (513, 2500, 1501, 1, -2.0, 0.25),
           (1024, 4100, 520, 2, 1.0, 0.0), (1030, 2049, 1003, 5, 1.0, 1.0), (300, 500, 129, 1, 1.0, 0.0),
           (65, 130, 64, 0, 1.0, 1.0)]
@@ -166,3 +166,29 @@ def test_every_tile_on_copies(lib, orc, dev, cfg, splits):
             got.append(host(dC))
         u.assert_fp32_close(got[0], want, scale, K, f"{cfg} {M}x{N}x{K} splits={splits}")
         u.assert_bits_equal(got[0], got[1], f"{cfg} and {direct} {M}x{N}x{K} splits={splits}")
+
+
+CAPTURED = [(284, 2304, 3904), (512, 8192, 512), (200, 9000, 1000), (1024, 4100, 520), (1000, 2048, 4096),
+            (700, 1024, 4096), (846, 7552, 3840), (571, 2731, 3648), (640, 2714, 3170), (976, 3648, 1243),
+            (176, 8384, 3392)]
+
+
+@pytest.mark.parametrize("M,N,K", CAPTURED)
+def test_captured_bits_are_eager_bits(lib, orc, dev, M, N, K):
+    """The route (on copies, or under capture while staging) changes no bit."""
+    A, B = u.normal(orc, M * K, 1).reshape(M, K), u.normal(orc, K * N, 2, 0, 0.02).reshape(K, N)
+    dA, dB = dev_copy(A, dev), dev_copy(B, dev)
+    dC, dE = torch.full((M, N), float("nan"), device=dev), torch.full((M, N), float("nan"), device=dev)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    lib.gemm_bf16_f32in(M, N, K, 1.0, dA, K, dB, N, 0.0, dE, N, stream=s.cuda_stream)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        lib.gemm_bf16_f32in(M, N, K, 1.0, dA, K, dB, N, 0.0, dC, N, stream=s.cuda_stream)
+    want = host(dE)
+    for rep in range(3):
+        dC.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        u.assert_bits_equal(host(dC), want, f"replay {rep}")
