@@ -280,7 +280,7 @@ int dnnopt_hip_plan_gemm_bf16_copies(int M, int N, int K, dnnopt_plan* out, int*
     const bool copies = plan_bf16_copies(L, M, N, K, K, N, N, &cp);
     *operands = copies ? (cp.both ? 2 : 1) : 0;
     *out = copies ? cp.L.pub : L.pub;
-    if (copies) out->workspace_bytes = cp.bytes + cp.L.part_bytes;
+    if (copies) out->workspace_bytes = cp.bytes;
     return DNNOPT_OK;
 }
 
@@ -393,14 +393,17 @@ static int gemm_bf16_common(int fp32_inputs, int M, int N, int K, float alpha, c
         // Operands rounded once into workspace (k padded with zeros to a
         // multiple of 8) ahead of the tiles.  Without the workspace (under
         // capture, or when memory is short) the tiles below round both while
-        // staging.
+        // staging.  The launch's partials are in the same buffer: nothing is
+        // enqueued before all scratch is there, and the GEMM slot never grows
+        // past what a captured call of this size uses.
         if (char* ws = static_cast<char*>(optional_workspace(s, cp.bytes, kSlotBf16))) {
             uint16_t *ca = reinterpret_cast<uint16_t*>(ws), *cb = reinterpret_cast<uint16_t*>(ws + cp.a_bytes);
             st = finish_launch(launch_bf16_copy(static_cast<const float*>(A), lda, static_cast<const float*>(B), ldb, M,
                                                 N, K, ca, cp.lda, cp.both ? cb : nullptr, cp.ldb, cp.K, s));
             if (st != DNNOPT_OK) return st;
+            const ExtScratch ext{ws + cp.copy_bytes, cp.bytes - cp.copy_bytes};
             return run_tile(cp.L, 0, 0, ca, cp.lda, cp.both ? static_cast<const void*>(cb) : B, cp.both ? cp.ldb : ldb, C, ldc,
-                            M, N, cp.K, alpha, beta, s);
+                            M, N, cp.K, alpha, beta, s, nullptr, &ext);
         }
     }
     return run_tile(L, 0, 0, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, s);

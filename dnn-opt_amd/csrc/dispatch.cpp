@@ -1341,6 +1341,11 @@ static bool make_bf16_copies(const Launch& direct, int M, int N, int K, int lda,
         *kb_ = (int)staged_bk(k);
         return (!forced || k == forced_cfg) && same_sums(k, direct.cfg, splits, K);
     };
+    // All of a call's scratch is one buffer: the copies, then a split launch's
+    // partials (laid out as ExtScratch).
+    const auto scratch = [&](const Launch& l, size_t copies) {
+        return copies + (l.part_bytes > 0 ? kTicketBytes + l.part_bytes : 0);
+    };
     out->lda = (int)k8;
     double best = forced ? 1e30 : 0.90 * direct.est_us;
     bool found = false;
@@ -1348,14 +1353,16 @@ static bool make_bf16_copies(const Launch& direct, int M, int N, int K, int lda,
     // (MI355X, us, direct -> A with 3 to 6 splits: 608 x 2677 x 3968 70.4 ->
     // 61.1, 144 x 3885 x 3776 45.8 -> 41.6, 176 x 6464 x 3767 45.5 -> 45.3, but
     // 96 x 4160 x 3392 22.1 vs 23.4 and 94 x 3789 x 3520 20.9 vs 21.8).
-    if (a <= kOptionalBytes && (forced || splits <= 2 || M > 128)) {
+    if (forced || splits <= 2 || M > 128) {
         const TilePick t = best_wg_tile(kA16Model, M, N, K, shape, splits);
         const double us = t.us + (double)M * K * 6e-6 / 6.3;
-        if (t.s > 0 && us < 0.95 * best) {
-            out->L = staged_launch(kTileA16, t.cfg, splits, M, N);
+        const Launch l = t.s > 0 ? staged_launch(kTileA16, t.cfg, splits, M, N) : Launch{};
+        if (t.s > 0 && us < 0.95 * best && scratch(l, a) <= kOptionalBytes) {
+            out->L = l;
             out->both = false;
             out->K = K;
-            out->a_bytes = out->bytes = a;
+            out->a_bytes = out->copy_bytes = a;
+            out->bytes = scratch(l, a);
             best = us;
             found = true;
         }
@@ -1371,13 +1378,14 @@ static bool make_bf16_copies(const Launch& direct, int M, int N, int K, int lda,
             two = t.s > 0 ? staged_launch(kTileBF16, t.cfg, splits, M, N) : Launch{};
             two.est_us = t.us;
         }
-        if (two.family == DNNOPT_K_TILE_BF16 && copy_us + two.est_us < 0.9 * best) {
+        if (two.family == DNNOPT_K_TILE_BF16 && copy_us + two.est_us < 0.9 * best && scratch(two, a + b) <= kOptionalBytes) {
             out->L = two;
             out->both = true;
             out->K = (int)k8;
             out->ldb = (int)n8;
             out->a_bytes = a;
-            out->bytes = a + b;
+            out->copy_bytes = a + b;
+            out->bytes = scratch(two, a + b);
             found = true;
         }
     }

@@ -144,7 +144,7 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
 int plan_s8(int epi, int M, int N, int K, Launch* L, bool lds_ok = true, int lda = 0, int ldb = 0, int ldc = 0);
 
 // Caller-provided device scratch in place of the stream's workspace: the
-// first kMaxTickets * 4 bytes are the ticket counters (zero between
+// first kTicketBytes are the ticket counters (zero between
 // launches), the rest holds partial sums.  A launch that needs more than
 // `bytes` fails with DNNOPT_ERR_SCRATCH_LIMIT; nothing is allocated.
 struct ExtScratch {
@@ -170,14 +170,15 @@ int plan_sgemm(int transA, int transB, int M, int N, int K, int lda, int ldb, La
 int plan_bf16(int fp32_inputs, int M, int N, int K, int lda, int ldb, Launch* L, int transB = 0, int ldc = 0);
 
 // The fp32-input bf16 GEMM with operands rounded to bf16 into workspace ahead
-// of the tiles: A alone (k_pp.hip's tiles round the fp32 B) or both (the
-// bf16-storage tiles).  Row strides and k of the copies in elements; false
-// where the tiles that round while staging are estimated faster, or the
-// copies may not be made.
+// of the tiles: A alone (k_tile.hip's kTileA16 tiles round the fp32 B while
+// staging it) or both (the bf16-storage tiles).  Row strides and k of the
+// copies in elements; false where the tiles that round both while staging are
+// estimated faster, or the copies may not be made.
 struct Bf16Copies {
     bool both;
     int lda, ldb, K;
-    size_t a_bytes, bytes;
+    size_t a_bytes, copy_bytes;  // A's copy, both copies
+    size_t bytes;                // all scratch: copies, ticket block, partials
     Launch L;
 };
 bool plan_bf16_copies(const Launch& direct, int M, int N, int K, int lda, int ldb, int ldc, Bf16Copies* out);

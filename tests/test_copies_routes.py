@@ -29,3 +29,24 @@ def test_copies_keep_the_splits(lib):
         made += p["operands"] > 0
         assert p["splits"] == lib.plan_bf16(M, N, K, fp32_inputs=1)["splits"], (M, N, K, p)
     assert made > 300
+
+
+def test_scratch_of_a_launch_on_copies(lib):
+    """The workspace of a launch on copies holds its split-k partials too, and
+    all of it stays within 256 MiB."""
+    rng = random.Random(2)
+    size = lambda lo, hi: int(lo * (hi / lo) ** rng.random())
+    pad = lambda v, n: (v + n - 1) // n * n
+    split = 0
+    for _ in range(3000):
+        M, N, K = size(65, 8192), size(768, 16384), size(768, 8192)
+        p = lib.plan_bf16_copies(M, N, K)
+        if not p["operands"]:
+            continue
+        copies = 2 * pad(K, 8) * (M + (pad(N, 8) if p["operands"] == 2 else 0))
+        tiles = pad(M, p["rows"]) * pad(N, p["cols"])
+        partials = 4 * p["splits"] * tiles if p["splits"] > 1 else 0
+        split += partials > 0
+        assert copies + partials <= p["workspace_bytes"] <= 256 << 20, (M, N, K, p)
+        assert p["workspace_bytes"] - copies - partials < (2 << 20), (M, N, K, p)
+    assert split > 50
