@@ -27,9 +27,10 @@ constexpr size_t kTicketBytes = (size_t)kMaxTickets * kTicketStride * sizeof(uns
 int get_workspace(hipStream_t s, size_t part_bytes, void** part, unsigned** tickets, int slot = 0);
 
 // Scratch of a slot for an optional faster route, without tickets and kept
-// like get_workspace's, at most kOptionalBytes per (device, stream).  nullptr
-// while the stream is being captured and when memory is short: the caller
-// takes its other route.
+// like get_workspace's, at most kOptionalBytes (a power of two) per (device,
+// stream); it grows to the next power of two, which waits for the stream.
+// nullptr while the stream is being captured and when memory is short: the
+// caller takes its other route.
 constexpr size_t kOptionalBytes = (size_t)256 << 20;
 void* optional_workspace(hipStream_t s, size_t bytes, int slot);
 

@@ -172,8 +172,12 @@ void* optional_workspace(hipStream_t s, size_t bytes, int slot) {
         }
     }
     if (e == hipSuccess) {
-        e = hipMalloc(&w->ptr, bytes);
-        if (e == hipSuccess) w->cap = bytes;
+        // Powers of two, so that a program whose sizes creep up waits and
+        // reallocates a few times in all, not at every larger call.
+        size_t cap = (size_t)1 << 20;
+        while (cap < bytes) cap *= 2;
+        e = hipMalloc(&w->ptr, cap);
+        if (e == hipSuccess) w->cap = cap;
         else w->ptr = nullptr;
     }
     if (e != hipSuccess) (void)hipGetLastError();

@@ -108,8 +108,14 @@ int dnnopt_hip_gemm_bf16_ex(int transA, int transB, int M, int N, int K,
                             const uint16_t* B, int ldb,
                             float beta, float* C, int ldc, void* stream);
 
-/* fp32 storage, both operands rounded to bf16 (nearest even) in registers,
- * fp32 accumulation.  Replaces dnnopt::gemm_bf16 (src/gemm/gemm.cpp:379-416). */
+/* fp32 storage, both operands rounded to bf16 (nearest even), fp32
+ * accumulation.  Replaces dnnopt::gemm_bf16 (src/gemm/gemm.cpp:379-416).
+ * Calls with more than 64 rows may round A, or both operands, ahead of the
+ * GEMM into library workspace (dnnopt_hip_plan_gemm_bf16_copies): at most
+ * 256 MiB per device and stream, kept until the process ends.  It grows in
+ * powers of two; a call that grows it waits for the stream first.  Captured
+ * calls, and calls that find no memory for it, round while staging instead,
+ * with the same bits. */
 int dnnopt_hip_gemm_bf16_f32in(int M, int N, int K,
                                float alpha, const float* A, int lda,
                                const float* B, int ldb,

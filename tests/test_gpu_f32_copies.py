@@ -192,3 +192,23 @@ def test_captured_bits_are_eager_bits(lib, orc, dev, M, N, K):
         torch.cuda.synchronize()
         g.replay()
         u.assert_bits_equal(host(dC), want, f"replay {rep}")
+
+
+def test_workspace_grows_in_powers_of_two(lib, dev):
+    """Sizes that creep up reallocate the copies' workspace a few times in all."""
+    s = torch.cuda.Stream()
+    N, K = 4096, 4096
+    plans = {M: lib.plan_bf16_copies(M, N, K) for M in range(960, 8192, 256)}
+    rows = [M for M, p in plans.items() if p["operands"] == 2 and p["splits"] == 1]
+    assert len(rows) > 8 and plans[rows[-1]]["workspace_bytes"] > 80 << 20, plans
+    B = torch.zeros((K, N), device=dev)
+    held = []
+    A, C = torch.zeros((max(rows), K), device=dev), torch.zeros((max(rows), N), device=dev)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    for M in rows:
+        lib.gemm_bf16_f32in(M, N, K, 1.0, A, K, B, N, 0.0, C, N, stream=s.cuda_stream)
+        torch.cuda.synchronize()
+        held.append(before - torch.cuda.mem_get_info()[0])
+        assert held[-1] >= plans[M]["workspace_bytes"]
+    assert len(set(held)) <= 3, held  # up to 128 MiB from 32 MiB at the least
