@@ -708,6 +708,7 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
         // while staging, in the same blocks of k.
         if (mode == kTileF2B && tile_a16(forced_cfg)) cfg = forced_cfg == kTileA16Tall && tall_ok ? kTileF2BTall : 20;
         if (mode == kTileF2B && tile_pp(forced_cfg) && tall_ok) cfg = kTileF2BTall;
+        if (mode == kTileF2B && forced_cfg == kTileF2BRaw) cfg = kTileF2BRaw;
         if (((forced_cfg >= kTileFirstLds && forced_cfg < kTileF32Few) || forced_cfg == kTileBF16Tb48 ||
              forced_cfg == kTileBF16Tb48Few || forced_cfg == kTileBF16Dma4w ||
              (tile_pp(forced_cfg) && mode == kTileBF16 && K % 8 == 0 && tall_ok) || (forced_cfg == kTileF2BTall && tall_ok)) &&
@@ -851,6 +852,12 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
     if (s > nblk) s = nblk;
     if (!span_ok(s)) return DNNOPT_ERR_UNSUPPORTED;
     if (tm > 65535 || s > 65535 || tn * tm > 0x7FFFFFF0ll) return DNNOPT_ERR_UNSUPPORTED;
+    // fp32 inputs on 32 x 64 tiles: operands kept unrounded in the register
+    // ring where every workgroup has a CU to itself and 8 blocks or more (with
+    // fewer, its longer start costs 3-4%; figures at dnnopt_tile_bf16_lds).
+    if (mode == kTileF2B && cfg == 19 && forced_cfg != 19 && (long long)xcd_grid((int)tn, (int)tm) * s <= cus &&
+        K / kb / s >= 8)
+        cfg = kTileF2BRaw;
     L->mode = mode;
     L->cfg = cfg;
     L->est_us = est_us;

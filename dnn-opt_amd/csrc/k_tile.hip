@@ -1370,6 +1370,7 @@ static const TileConfig kTileConfigs[] = {
     // bf16 A, fp32 B (kTileA16): {MT, NT, WM, WN, 1, depth, k per block}
     {2, 3, 4, 2, 1, 2, 128},  // 65: 128 x 96
     {4, 3, 4, 2, 1, 2, 64},   // 66: 256 x 96
+    {2, 1, 1, 4, 1, 3, 128},  // 67: 32 x 64, fp32 inputs unrounded in the register ring
 };
 
 int tile_config_count() { return (int)(sizeof(kTileConfigs) / sizeof(kTileConfigs[0])); }
@@ -1459,9 +1460,8 @@ hipError_t launch_tile(int mode, int cfg_idx, int ta, int tb, int al, dim3 grid,
         q.tiles_m = a.tiles_m;
         return launch_pp(0, cfg_idx - kTilePPFirst, tb, 0, grid, q, s);
     }
-    if (cfg_idx == 19 && mode == kTileF2B && (long long)grid.x * grid.z <= 256 && a.K / 128 / a.splits >= 8) {
-        // a CU to every workgroup and 8 blocks or more each (with fewer, its
-        // longer start costs 3-4%): the raw ring (see dnnopt_tile_bf16_lds)
+    if (cfg_idx == kTileF2BRaw) {
+        if (mode != kTileF2B || !al) return hipErrorInvalidValue;
         hipLaunchKernelGGL((dnnopt_tile_bf16_lds<2, 1, 1, 4, 3, kTileF2B, 0, 128, 1, 1>), grid, dim3(256), 0, s, a);
         return hipGetLastError();
     }

@@ -271,6 +271,9 @@ constexpr bool tile_wavek(int cfg) { return cfg >= kTileWavekFirst && cfg <= kTi
 // configurations 20 and kTileF2BTall.
 constexpr int kTileA16Wide = 65, kTileA16Tall = 66;
 constexpr bool tile_a16(int cfg) { return cfg == kTileA16Wide || cfg == kTileA16Tall; }
+// fp32 inputs, the 32 x 64 tiles of configuration 19 with operands unrounded in
+// the register ring (RAW in k_tile.hip).
+constexpr int kTileF2BRaw = 67;
 constexpr bool tile_f32_dma(int cfg) { return cfg >= kTileF32DmaFirst && cfg <= kTileF32DmaLast; }
 // k per LDS block of an LDS-staged configuration: its kblk (or
 // DNNOPT_LDS_KB) when both stages fit in 128 KiB of LDS, else 64.

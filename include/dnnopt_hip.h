@@ -319,7 +319,8 @@ int dnnopt_hip_device_count(void);    /* 0 when no device is visible        */
                                            fp32 register tiles: 1-4, 35, 36; fp32 LDS-DMA tiles,
                                            A stored M x K: 41-47, and 48-50 with B stored N x K;
                                            four waves splitting k: 58-64; bf16 from fp32 inputs
-                                           on copies of both operands: 51-57, of A: 65, 66) */
+                                           on copies of both operands: 51-57, of A: 65, 66, 32 x
+                                           64 tiles rounding late: 67) */
 #define DNNOPT_TUNE_TILE_TICKET     11
 #define DNNOPT_TUNE_S8_CFG          12
 #define DNNOPT_TUNE_S8_ROWDOT       13

@@ -212,3 +212,25 @@ def test_workspace_grows_in_powers_of_two(lib, dev):
         held.append(before - torch.cuda.mem_get_info()[0])
         assert held[-1] >= plans[M]["workspace_bytes"]
     assert len(set(held)) <= 3, held  # up to 128 MiB from 32 MiB at the least
+
+
+@pytest.mark.parametrize("M,N,K", [(9, 64, 1), (32, 70, 1023), (31, 4096, 1024), (16, 16384, 1024), (33, 130, 1152),
+                                   (64, 8192, 1300)])
+@pytest.mark.parametrize("splits", [1, 2])
+def test_32_row_tiles_rounding_early_or_late(lib, orc, dev, M, N, K, splits):
+    """The 32 x 64 tiles round an operand when it arrives (TILE_CFG 19) or when
+    it is written to LDS (67): the same bits, on both sides of the rule that
+    picks between them (a CU to every workgroup, 8 blocks of 128 k or more)."""
+    A, B = u.normal(orc, M * K, 1).reshape(M, K), u.normal(orc, K * N, 2, 0, 0.02).reshape(K, N)
+    dA, dB = dev_copy(A, dev), dev_copy(B, dev)
+    got = []
+    for cfg in (19, 67):
+        dC = torch.full((M, N), float("nan"), device=dev)
+        with lib.tunables(TILE_CFG=cfg, TILE_SPLITS=splits):
+            p = lib.plan_bf16(M, N, K, fp32_inputs=1)
+            assert (p["rows"], p["cols"], p["block"]) == (32, 64, 256), p
+            lib.gemm_bf16_f32in(M, N, K, 1.0, dA, K, dB, N, 0.0, dC, N, stream=stream())
+        got.append(host(dC))
+    want, scale = u.exact(u.bf16_value(u.bf16_bits(orc, A)), u.bf16_value(u.bf16_bits(orc, B)))
+    u.assert_fp32_close(got[1], want, scale, K, f"{M}x{N}x{K} splits={splits}")
+    u.assert_bits_equal(got[0], got[1], f"{M}x{N}x{K} splits={splits}")
