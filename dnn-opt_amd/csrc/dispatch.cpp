@@ -891,8 +891,8 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
     L->tickets = (s > 1 && !L->defer_reduce) ? (int)tiles : 0;
     const int kernel = mode == kTileF32 ? DNNOPT_K_TILE_F32 : DNNOPT_K_TILE_BF16;
     fill_pub(L, kernel,
-             mode == kTileF32 ? (f32dma ? "dnnopt_tile_f32_dma" : "dnnopt_tile_f32")
-                              : (dma ? "dnnopt_tile_bf16_dma" : (lds ? "dnnopt_tile_bf16_lds" : "dnnopt_tile_bf16")),
+             mode == kTileF32 ? (f32dma ? "dnnopt_tile_f32_dma" : "dnnopt_tile_f32")  // (a prefix of k_wavek.hip's too)
+                              : (tile_pp(cfg) ? "dnnopt_tile_bf16_dma_pp" : dma ? "dnnopt_tile_bf16_dma" : (lds ? "dnnopt_tile_bf16_lds" : "dnnopt_tile_bf16")),
              bm, bn, (int)s, waves_per_wg * 64);
     return DNNOPT_OK;
 }
@@ -1005,7 +1005,7 @@ static int plan_s8_kernels(int epi, int M, int N, int K, Launch* L, bool lds_ok,
     L->grid = lds ? dim3((unsigned)xcd_grid((int)tn, (int)tm), 1, (unsigned)s) : dim3((unsigned)tn, (unsigned)tm, (unsigned)s);
     L->part_bytes = s > 1 ? (size_t)s * tiles * bm * bn * sizeof(int32_t) : 0;
     L->tickets = (s > 1 && !L->defer_reduce) ? (int)tiles : 0;
-    fill_pub(L, DNNOPT_K_MFMA_S8, dma ? "dnnopt_s8_dma" : (lds ? "dnnopt_s8_lds" : "dnnopt_mfma_s8"), bm, bn, (int)s,
+    fill_pub(L, DNNOPT_K_MFMA_S8, cfg >= kS8PPFirst ? "dnnopt_s8_dma_pp" : dma ? "dnnopt_s8_dma" : (lds ? "dnnopt_s8_lds" : "dnnopt_mfma_s8"), bm, bn, (int)s,
              waves_per_wg * 64);
     return DNNOPT_OK;
 }
@@ -1287,7 +1287,7 @@ static Launch staged_launch(int mode, int cfg, long long s, int M, int N) {
     L.grid = dim3((unsigned)xcd_grid(L.tn, L.tm), 1, (unsigned)s);
     L.defer_reduce = s > 1 ? 1 : 0;
     L.part_bytes = s > 1 ? (size_t)s * L.tn * L.tm * L.bm * L.bn * sizeof(float) : 0;
-    fill_pub(&L, DNNOPT_K_TILE_BF16, tile_pp(cfg) ? "dnnopt_tile_bf16_dma" : "dnnopt_tile_bf16_lds", L.bm, L.bn, (int)s,
+    fill_pub(&L, DNNOPT_K_TILE_BF16, tile_pp(cfg) ? "dnnopt_tile_bf16_dma_pp" : "dnnopt_tile_bf16_lds", L.bm, L.bn, (int)s,
              c.wm * c.wn * c.kw * 64);
     return L;
 }

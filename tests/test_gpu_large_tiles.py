@@ -124,6 +124,16 @@ def test_planned_by_size_and_k_alignment(lib):
             assert (p["rows"], p["cols"]) not in large, p
 
 
+def test_plans_name_the_kernel(lib):
+    """A plan's name is the kernel's, not that of the kernel it stands in for."""
+    assert lib.plan_bf16_ex(2048, 11008, 4096, transB=1)["name"] == "dnnopt_tile_bf16_dma_pp"
+    assert lib.plan_bf16_copies(1024, 11008, 4096)["name"] == "dnnopt_tile_bf16_dma_pp"
+    assert lib.plan_s8(1024, 11008, 4096)["name"] == "dnnopt_s8_dma_pp"
+    with lib.tunables(TILE_CFG=33, S8_CFG=29):
+        assert lib.plan_bf16_ex(2048, 11008, 4096, transB=1)["name"] == "dnnopt_tile_bf16_dma"
+        assert lib.plan_s8(1024, 11008, 4096)["name"] == "dnnopt_s8_dma"
+
+
 @pytest.mark.parametrize("M,N,K", [(4096, 4096, 8400000), (2048, 1024, 8400000), (1024, 1024, 17000000),
                                    (256, 64, 8388608), (2048, 4096, 16777200), (128, 128, 16777216)])
 def test_int8_long_rows_keep_tiles(lib, M, N, K):
