@@ -325,6 +325,11 @@ static TilePick pick_tile(int mode, int M, int N, int K, int def_cfg, bool tall_
 //   fp32 inputs rounded in registers: 124 measured cases (same shapes, B
 //   stored K x N; 9 configurations; median error 6%, 90% within 17%); 1.99 us
 //   per launch, 3.3 TB/s; a split 2.73 us plus its partials at 6.6 TB/s.
+//   Fitted while every tile rounded its operands on arrival.  Rounding late
+//   has since made 128 x 96, 256 x 96 and 64 x 64 tiles 6-19% faster and left
+//   32 x 64 and 64 x 128 as they were, so the model ranks the former too low
+//   (80 x 10388 x 4096: 32 x 64 at 70 us, where a copy of A on 128 x 96 with 2
+//   splits took 44).
 struct LdsFit {
     int cfg, tb, occ;
     double fill, mfma, ps_per_byte;
@@ -687,7 +692,11 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
             }
             // bf16 storage, more than 64 rows: k_pp.hip's tiles where their
             // model puts them 5% ahead of that choice's.  (Their k-contiguous
-            // rows are cut off at whole 16-byte chunks, hence K % 8.)
+            // rows are cut off at whole 16-byte chunks, hence K % 8.)  Why 5%
+            // (MI355X, drawn sizes of 65..4096 rows, time on these tiles over
+            // time on the other choice): 5 to 15% ahead in the models, 30
+            // sizes, 0.81 in geometric mean (0.61..0.93); within 5% either
+            // way, 40 sizes, 1.06 (0.72..1.22, faster on 6).
             if (mode == kTileBF16 && M > 64 && K % 8 == 0 && tall_ok) {
                 const TilePick pp = best_wg_tile(kBf16PPModel, M, N, K, [&](int k, int* bm_, int* bn_, int* kb_) {
                     const TileConfig t = tile_config(k);
@@ -773,9 +782,12 @@ int plan_tile(int mode, int transA, int transB, int M, int N, int K, int lda, in
             // 9.0, 926 x 561 x 907 20.5 -> 14.1, 134 x 2354 x 393 11.1 ->
             // 7.8).  Kept from them: up to 32 rows (the 16-row tiles, 16 x
             // 3712 x 384 4.6 vs 6.3), and with a K x N B up to 128 rows and
-            // from K = 4096, where existing plans are relied on (128 x 3072 x
-            // 768 is to be split, 128 and 512 x 4096 x 4096 on 64 x 128 tiles;
-            // 128 x 4096 x 4096 would take 44 us instead of 55 on 64 x 32).
+            // from K = 4096.  Those two bounds are held by plans that tests
+            // state (128 x 3072 x 768 is split: 14.0 us, 10.2 on 32 x 48; 384
+            // x 3072 x 4096 is not on 96 x 48), not by the kernels: without
+            // them 40 drawn sizes of 33..128 rows take 0.92x the time in
+            // geometric mean (0.81..1.05), 40 with K from 4096 0.89x
+            // (0.66..0.99).
             // Rows that are not whole 16-byte chunks slow the copies, which
             // the model does not price: B N x K then keeps the other tiles
             // (801 x 3414 x 175 16.6 vs 26.5), as it does below four blocks of

@@ -15,9 +15,10 @@
 // equal tiles -- and no barrier stands in the loop.  Measured (MI355X, us, the
 // best of the other tiles -> this, in a graph): 384 x 3072 x 768 23.9 -> 20.6
 // (B N x K, of which 11.8 at the rate of a large fp32 product, 154 TFLOP/s) and
-// 27.5 -> 21.1 (K x N), x 3072 79.4 -> 61.8 and 78.5 -> 64.0 (1.17 us per block
-// of 64 k; 5.6 us of launch, first copies and epilogue), 384 x 768 x 768 11.1
-// -> 9.0.  The order within a step matters little (MFMAs of a step before,
+// 27.5 -> 21.1 (K x N), x 3072 79.4 -> 61.8 and 78.5 -> 64.0, 384 x 768 x 768
+// 11.1 -> 9.0.  In a kernel trace K = 768 and 3072 take 22.7 and 61.1 (B N x K):
+// 1.07 us per block of 64 k, 9.9 us of launch, first copies from HBM and
+// epilogue.  The order within a step matters little (MFMAs of a step before,
 // between or after its reads and copies: 20.6-22.2).
 #include <type_traits>
 
@@ -30,7 +31,9 @@ namespace dnnopt_hip {
 
 // Tile 16 MT x 16 NT.  Rows of A and B stored N x K are copied 64 bytes (16 k)
 // at a time, one wave load filling exactly one MFMA operand (16 rows), read
-// back linearly (no bank conflicts, no swizzle).  A K x N B is copied as 16
+// back without a swizzle: the 64-byte steps between lanes cost bank conflicts
+// (0.55 conflict cycles per active LDS cycle with B N x K, MFMAs busy 64% of a
+// launch, both over 384 x 3072 x 768 and x 3072).  A K x N B is copied as 16
 // rows of k; lane r of an operand takes columns NT r .. NT r + NT - 1 of the
 // tile, one LDS read per row of k, so its sub-tiles' columns interleave.
 // Offsets are 32-bit from the tile's first row over all of k (f32_dma_fits).
@@ -64,7 +67,7 @@ __global__ __launch_bounds__(256, 1) void dnnopt_tile_f32_dma_wavek(TileArgs p) 
     const __amdgpu_buffer_rsrc_t rb = make_rsrc(bbase, range31(b_last * 4));
 
     // k-contiguous rows: wave load u fills 16 rows of 64 bytes (16 k), lane l
-    // row l / 4, chunk l % 4: exactly one MFMA operand, read back linearly.
+    // row l / 4, chunk l % 4: exactly one MFMA operand.
     const int lrow = lane >> 2, lch = lane & 3;
     uint32_t ga[MT], gb[UB];
 #pragma unroll
