@@ -229,7 +229,8 @@ def kernel_key(lib, case):
         if p["name"] == "dnnopt_skinny_q8":
             return f"dnnopt_skinny_q8<{case.M}>", p
         if p["name"] == "dnnopt_s8_lds_q8b":
-            return "dnnopt_s8_lds<2, 1, 2, 2, 3, 1, 128, 1>", p
+            # 64 x 32 tiles: two wave groups sharing k, or one
+            return "dnnopt_s8_lds<2, 1, 2, 2, %s>" % ("2, 1, 128, 1, 2" if p["block"] == 512 else "3, 1, 128, 1, 1"), p
     else:
         p = lib.plan_s8(case.M, case.N, case.K, with_scale=int(case.kind == "s8s"))
     if p["name"] == "dnnopt_skinny":

@@ -1342,7 +1342,7 @@ static bool same_sums(int cfg1, int cfg2, long long s, int K) {
 static bool make_bf16_copies(const Launch& direct, int M, int N, int K, int lda, int ldb, int ldc, Bf16Copies* out) {
     if (ldc <= 0) ldc = N;
     const int forced_cfg = tunable(kTuneTileCfg);
-    const bool force_a = tile_a16(forced_cfg), force_both = tile_pp(forced_cfg), forced = force_a || force_both;
+    const bool forced = tile_a16(forced_cfg) || tile_pp(forced_cfg);
     if (direct.mode != kTileF2B || direct.cfg < kTileFirstLds || direct.family != DNNOPT_K_TILE_BF16) return false;
     if ((!forced && (direct.est_us <= 0.0 || M <= 64)) || (long long)lda * 16 >= 0x7FFFFFFFll ||
         (long long)ldb * 16 >= 0x7FFFFFFFll)

@@ -83,3 +83,14 @@ def test_counter_files_name_a_traced_kernel():
         traces = glob.glob(os.path.join(u.ROOT, "profiles", f"*_{wl}_kernel_trace.txt"))
         assert traces, f
         assert any(inst in open(t).read() for t in traces), (f, inst)
+
+
+def test_fp32_api_int8_kernel_is_the_traced_one(lib):
+    """The kernel named for the 128-row fp32-API int8 case is the instance its
+    trace lists, and its traffic figure is found."""
+    case = [c for c in bench.workload("c5f")[1] if c.M == 128][0]
+    key, plan = bench.kernel_key(lib, case)
+    trace = open(os.path.join(u.ROOT, "profiles", "dnnopt_s8_lds_q8b_64x32_c5f_kernel_trace.txt")).read()
+    row = [l for l in trace.splitlines() if l.startswith(key + " ")]
+    assert row and int(row[0][len(key):].split()[1]) == plan["block"], key
+    assert bench.read_traffic(key, "c5f")
